@@ -27,6 +27,7 @@ namespace {
 
 constexpr int kWave = 64;
 constexpr int kThreads = 256;
+constexpr int kMaxBlocks = 1 << 23; // of kThreads threads in one launch: a launch holds fewer than 2^32 threads
 constexpr int kChunk = 64;      // positions per attention block
 constexpr int kMaxHeadDim = 256;
 constexpr int kMaxGroup = 16;   // query heads per KV head
@@ -183,10 +184,13 @@ __global__ __launch_bounds__(kThreads) void rope_kv_rows(float *__restrict__ q, 
   }
 }
 
-// rope_kv_rows for head_dim HD = 64 or 128: thread (row, d4) takes dimensions 4 d4 .. 4 d4 + 3 of every head of its
-// row (q heads, then k, then v), so the row's table values for them are loaded once and all of its loads are in
-// flight together; each element gets the same products in the same order as in rope_kv_rows, so the results are
-// bitwise those of rope_kv_rows.
+// rope_kv_rows for head_dim HD = 64 or 128: thread (row, d4) of a unit takes dimensions 4 d4 .. 4 d4 + 3 of two q heads
+// of its row, or of one KV head (k and v), its loads in flight together and the row's table values loaded once for
+// them. Each element gets the same products in the same order as in rope_kv_rows, so the results are bitwise those of
+// rope_kv_rows. Latency bounds it until the rows are many, then the memory: 2 rows of 32 + 8 heads of 128 take 2.4 us,
+// 256 rows 4.1 us (3.4 TB/s) and 2048 rows 19.9 us (5.5 TB/s) where a thread that walked every head of its row, each
+// load behind the one before, took 7.7, 10.1 and 20.4 us. A block's neighbours take the next heads of the same rows,
+// not the next rows of the same heads: the latter, a row's stride apart, ran 256 rows in 12 us.
 template <int HD>
 __global__ __launch_bounds__(kThreads) void rope_kv_rows_hd(float *__restrict__ q, size_t q_stride, float *__restrict__ k,
                                                             const float *__restrict__ v, size_t kv_stride,
@@ -196,24 +200,31 @@ __global__ __launch_bounds__(kThreads) void rope_kv_rows_hd(float *__restrict__ 
                                                             float *__restrict__ value_cache, int pos0,
                                                             size_t pos_stride, size_t head_base) {
   constexpr int hd4 = HD / 4, kRowsPerBlock = kThreads / hd4;
-  const int r = blockIdx.x * kRowsPerBlock + threadIdx.x / hd4, d = 4 * (threadIdx.x % hd4);
+  const int qunits = (n_heads + 1) / 2, units = qunits + n_kv_heads;
+  const int unit = blockIdx.x % units;
+  const int r = blockIdx.x / units * kRowsPerBlock + threadIdx.x / hd4, d = 4 * (threadIdx.x % hd4);
   if (r >= rows)
     return;
-  const Rot4 rot = rot4_of(table + (size_t)r * table_stride, HD, d);
-  float *qr = q + (size_t)r * q_stride + d;
-  for (int h = 0; h < n_heads; h++) {
-    float4 *pq = reinterpret_cast<float4 *>(qr + (size_t)h * HD);
-    *pq = rotate4(*pq, rot);
+  const float *t = table + (size_t)r * table_stride;
+  if (unit < qunits) {
+    float4 *pq = reinterpret_cast<float4 *>(q + (size_t)r * q_stride + (size_t)(2 * unit) * HD + d);
+    const bool two = 2 * unit + 1 < n_heads;
+    const float4 x0 = pq[0], x1 = pq[two ? hd4 : 0];
+    const Rot4 rot = rot4_of(t, HD, d);
+    pq[0] = rotate4(x0, rot);
+    if (two)
+      pq[hd4] = rotate4(x1, rot);
+    return;
   }
-  const size_t slot0 = (size_t)(pos0 + r) * pos_stride + d;
-  for (int g = 0; g < n_kv_heads; g++) {
-    const size_t at = (size_t)r * kv_stride + (size_t)g * HD + d, slot = slot0 + (size_t)g * head_base;
-    float4 *pk = reinterpret_cast<float4 *>(k + at);
-    const float4 x = rotate4(*pk, rot);
-    *pk = x;
-    *reinterpret_cast<float4 *>(key_cache + slot) = x;
-    *reinterpret_cast<float4 *>(value_cache + slot) = *reinterpret_cast<const float4 *>(v + at);
-  }
+  const int g = unit - qunits;
+  const size_t at = (size_t)r * kv_stride + (size_t)g * HD + d;
+  const size_t slot = (size_t)(pos0 + r) * pos_stride + (size_t)g * head_base + d;
+  float4 *pk = reinterpret_cast<float4 *>(k + at);
+  const float4 x = *pk, y = *reinterpret_cast<const float4 *>(v + at);
+  const float4 z = rotate4(x, rot4_of(t, HD, d));
+  *pk = z;
+  *reinterpret_cast<float4 *>(key_cache + slot) = z;
+  *reinterpret_cast<float4 *>(value_cache + slot) = y;
 }
 
 // ---- embedding rows -------------------------------------------------------------------------------------------------
@@ -234,6 +245,29 @@ __global__ __launch_bounds__(kThreads) void embed_rows(float *__restrict__ out, 
   }
   const size_t at = (size_t)id * dim + j;
   out[(size_t)r * dim + j] = (float)table[at] * scales[at / gs];
+}
+
+// The same for dim and gs multiples of 4 and aligned operands: four values of one scale per thread, per_row blocks a
+// row. The write of the rows bounds it: 2048 ids of 4096 values take 9.3 us (4.5 TB/s), where one value a thread behind
+// two 64-bit divisions took 20.6 us; 256 ids 3.2 us, before 4.2.
+__global__ __launch_bounds__(kThreads) void embed_rows4(float *__restrict__ out, const int8_t *__restrict__ table,
+                                                        const float *__restrict__ scales, const int *__restrict__ ids,
+                                                        unsigned per_row, unsigned dim, unsigned gs, int vocab,
+                                                        int *flags) {
+  const unsigned r = blockIdx.x / per_row, j = 4 * (blockIdx.x % per_row * kThreads + threadIdx.x);
+  if (j >= dim)
+    return;
+  const int id = ids[r];
+  if (id < 0 || id >= vocab) {
+    flags[2] = 1;
+    return;
+  }
+  const size_t at = (size_t)id * dim + j;
+  // where whole groups fill a row the quotient needs 32 bits only
+  const float s = scales[dim % gs ? at / gs : (size_t)id * (dim / gs) + j / gs];
+  const char4 w = *reinterpret_cast<const char4 *>(table + at);
+  *reinterpret_cast<float4 *>(out + (size_t)r * dim + j) =
+      float4{(float)w.x * s, (float)w.y * s, (float)w.z * s, (float)w.w * s};
 }
 
 // The FP32 table's lookup (src/tp.c:342 for a token, 449 for a batch): a copy of row ids[i], 16 bytes per thread when
@@ -1514,14 +1548,18 @@ bool launch_rope_kv_rows(float *q, size_t q_stride, float *k, const float *v, si
                          float *value_cache, int pos0, size_t pos_stride, size_t head_base, hipStream_t stream) {
   const int per_row = (n_heads + 2 * n_kv_heads) * (head_dim / 4);
   if (head_dim == 128 || head_dim == 64) {
-    const int rows_per_block = kThreads / (head_dim / 4);
-    const dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block));
-    if (head_dim == 128)
-      hipLaunchKernelGGL(rope_kv_rows_hd<128>, grid, dim3(kThreads), 0, stream, q, q_stride, k, v, kv_stride, table,
-                         table_stride, rows, n_heads, n_kv_heads, key_cache, value_cache, pos0, pos_stride, head_base);
-    else
-      hipLaunchKernelGGL(rope_kv_rows_hd<64>, grid, dim3(kThreads), 0, stream, q, q_stride, k, v, kv_stride, table,
-                         table_stride, rows, n_heads, n_kv_heads, key_cache, value_cache, pos0, pos_stride, head_base);
+    const int rows_per_block = kThreads / (head_dim / 4), units = (n_heads + 1) / 2 + n_kv_heads;
+    const int most = max(kMaxBlocks / units, 1) * rows_per_block; // rows of a launch
+    for (int r0 = 0; r0 < rows; r0 += most) {
+      const int n = min(most, rows - r0);
+      const dim3 grid((unsigned)((n + rows_per_block - 1) / rows_per_block) * (unsigned)units);
+      hipLaunchKernelGGL(head_dim == 128 ? rope_kv_rows_hd<128> : rope_kv_rows_hd<64>, grid, dim3(kThreads), 0, stream,
+                         q + (size_t)r0 * q_stride, q_stride, k + (size_t)r0 * kv_stride, v + (size_t)r0 * kv_stride,
+                         kv_stride, table + (size_t)r0 * table_stride, table_stride, n, n_heads, n_kv_heads, key_cache,
+                         value_cache, pos0 + r0, pos_stride, head_base);
+      if (rows - r0 <= most)
+        break;
+    }
     return launch_ok("rope_kv_rows_hd");
   }
   const long long threads = (long long)rows * per_row;
@@ -1541,6 +1579,13 @@ bool launch_kv_store(float *cache, const float *src, size_t src_ld, int pos0, in
 
 bool launch_embed_rows(float *out, const int8_t *table, const float *scales, const int *ids, int count, int dim,
                        int gs, int vocab, hipStream_t stream) {
+  const long long per_row = ((long long)dim + 4 * kThreads - 1) / (4 * kThreads);
+  if (dim % 4 == 0 && gs % 4 == 0 && ((uintptr_t)table & 3) == 0 && ((uintptr_t)out & 15) == 0 &&
+      count * per_row <= kMaxBlocks) {
+    hipLaunchKernelGGL(embed_rows4, dim3((unsigned)(count * per_row)), dim3(kThreads), 0, stream, out, table, scales, ids,
+                       (unsigned)per_row, (unsigned)dim, (unsigned)gs, vocab, device().error_flags);
+    return launch_ok("embed_rows4");
+  }
   const long long threads = (long long)count * dim;
   hipLaunchKernelGGL(embed_rows, dim3((unsigned)((threads + kThreads - 1) / kThreads)), dim3(kThreads), 0, stream, out,
                      table, scales, ids, count, dim, gs, vocab, device().error_flags);

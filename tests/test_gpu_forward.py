@@ -439,6 +439,25 @@ def test_attention_nonfinite_score_fails_and_bookkeeping():
 # ---- embedding rows ------------------------------------------------------------------------------------------------
 
 
+@pytest.mark.parametrize("dim,gs,shift", [(4, 4, 0), (1020, 60, 0), (1024, 64, 0), (1028, 4, 0), (2176, 128, 0),
+                                          (1026, 6, 0), (1024, 64, 1)])
+def test_embed_q8_rows_widths(dim, gs, shift):
+    """Widths on both sides of the 1024 values that a block of four values a thread takes, groups that fill rows and
+    that straddle them, and the one-value kernel (a dim that is no multiple of 4, a table at an odd address): bitwise
+    numpy's float32 product."""
+    L = hu.lib()
+    rng = np.random.default_rng(orc.SEED + 911 + dim + gs)
+    vocab = 2 * gs
+    table = rng.integers(-127, 128, vocab * dim + shift, dtype=np.int8)
+    scales = rng.uniform(1e-4, 2e-2, vocab * dim // gs).astype(np.float32)
+    ids = rng.integers(0, vocab, 9).astype(np.int32)
+    flat = ids[:, None].astype(np.int64) * dim + np.arange(dim)
+    want = table[shift:][flat].astype(np.float32) * scales[flat // gs]
+    dt, ds, di, do = hu.dev(table), hu.dev(scales), hu.dev(ids), hu.empty(len(ids) * dim, hu.torch().float32)
+    L.k_embed_q8_rows(lh.ptr(do), lh.ptr(dt[shift:]), lh.ptr(ds), lh.ptr(di), len(ids), dim, gs, vocab)
+    assert np.array_equal(hu.bits(hu.host(do)).reshape(len(ids), dim), hu.bits(want))
+
+
 def test_embed_q8_rows_bitwise_host_device_and_bad_id():
     """Embedding lookup of a Q8_0 table (src/tp.c:395-396, 444-456): each value is the int8 converted exactly times its
     group's scale, one float product, so the row is bitwise numpy's float32 product. Groups straddle rows (dim 96,
@@ -599,6 +618,32 @@ def test_rope_kv_store_rows_fused(rows, nh, nkv, hd, seq, pos0, layout):
         assert np.array_equal(out[0][0][0], hu.bits(wq)) and np.array_equal(out[0][1][0], hu.bits(wk))
     finally:
         L.kernels_kv_layout_select(b"head")
+
+
+@pytest.mark.parametrize("rows,nh,nkv,hd", [(1, 1, 1, 128), (7, 3, 3, 128), (8, 5, 1, 128), (9, 2, 2, 64), (17, 15, 3, 64)])
+def test_rope_kv_store_rows_head_counts(rows, nh, nkv, hd):
+    """The rows kernel of head_dim 64 and 128 takes two q heads or one KV head per unit: odd head counts, and rows on
+    both sides of a block's 8 or 16, bitwise the separate calls; the rows of the strides' padding stay untouched."""
+    L = hu.lib()
+    rng = orc.Rng(orc.SEED + 4700 + rows + nh + hd)
+    qs, ks, seq, pos0 = nh * hd + 8, nkv * hd + 4, rows + 5, 3
+    q, k, v = (rng.normal(rows * n, 0, 1).reshape(rows, n) for n in (qs, ks, ks))
+    table = rng.uniform(rows * 2 * hd, 1.0).reshape(rows, 2 * hd)
+    out = []
+    for fused in (True, False):
+        dq, dk, dv, dt = hu.dev(q), hu.dev(k), hu.dev(v), hu.dev(table)
+        dkc, dvc = hu.dev(np.zeros(seq * nkv * hd, np.float32)), hu.dev(np.zeros(seq * nkv * hd, np.float32))
+        if fused:
+            L.llhip_rope_kv_store_rows(lh.ptr(dq), qs, lh.ptr(dk), lh.ptr(dv), ks, lh.ptr(dt), 2 * hd, rows, nh, nkv, hd,
+                                       lh.ptr(dkc), lh.ptr(dvc), pos0, seq)
+        else:
+            L.k_rope_apply_rows(lh.ptr(dq), qs, lh.ptr(dk), ks, lh.ptr(dt), 2 * hd, rows, nh, nkv, hd)
+            L.k_kv_store(lh.ptr(dkc), lh.ptr(dk), ks, pos0, rows, nkv, hd, seq)
+            L.k_kv_store(lh.ptr(dvc), lh.ptr(dv), ks, pos0, rows, nkv, hd, seq)
+        assert lh.last_error() == "", lh.last_error()
+        out.append([hu.bits(hu.host(a)) for a in (dq, dk, dkc, dvc)])
+    for what, a, b in zip(("q", "k", "key cache", "value cache"), *out):
+        assert np.array_equal(a, b), what
 
 
 # ---- RoPE and the cache stores recorded into the decode attention ----------------------------------------------------
