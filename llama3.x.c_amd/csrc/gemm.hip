@@ -366,9 +366,16 @@ template <int N> __device__ __forceinline__ void wait_vmcnt_lgkm0() {
 
 // Split K: a grid with fewer tiles than CUs runs each tile as `splits` blocks over consecutive K ranges, each writing
 // its partial tile to a device workspace. The partials are added in split order, so results do not depend on timing:
-// by split_reduce, a second kernel (int8 and wide BF16 kernels, which have no registers to spare), or by the last of
-// the tile's blocks to arrive (split_combine, the FP32 / BF16 kernel), which counts the arrivals and puts the counter
-// back to zero.
+// by split_reduce, a second kernel (the int8 and wide BF16 kernels, and the FP32 / BF16 kernels from four splits), or
+// by the last of the tile's blocks to arrive (split_combine, the FP32 / BF16 kernels with two or three splits), which
+// counts the arrivals and puts the counter back to zero.
+//
+// The last block alone reads its tile's `splits` partials, 128 KB each, at one CU's rate while the others idle;
+// split_reduce reads them on every CU but is one more launch. Measured, last block / second kernel: two splits (64 x
+// 2 * 8192 x 3072 BF16) 37.7 / 40.3 us, three (512 x 5120 x 3072) 40.4 / 40.5, five (512 x 3072 x 3072) 43.8 / 32.4 and
+// (512 x 3072 x 8192) 80.9 / 56.3, ten (256 x 3072 x 3072) 45.0 / 26.0; FP32 three (333 x 5120 x 3072) 92.5 / 93.9, five
+// (333 x 3072 x 8192) 178 / 157, sixteen (100 x 2048 x 2048) 54.8 / 31.0.
+constexpr int kCombineSplits = 3;
 
 // Cache policy of the partial tiles' stores and loads: device-coherent (sc1), so a store is written through past the
 // XCD's L2 before its completion is counted, and a load reads from past it. No cache-wide write-back or invalidate is
@@ -421,10 +428,20 @@ __device__ __forceinline__ bool split_combine(const SplitK &sk, int tile, int sp
   return true;
 }
 
-// The second kernel of a split launch whose kernel wrote partial tiles (the int8 and the wide BF16 kernels): thread by
-// thread over every tile's partial sums. A thread takes one accumulator pair, tiles j and j + J/2 of row tile i of
-// one lane of the block layout (the SWIGLU pair, or two plain column tiles), adds the splits in order and applies the
-// epilogue to its four rows. Partial tile layout: [tile][split][i * J + j][THREADS] v4f.
+// A block's partial tile into its slot, for split_reduce.
+__device__ __forceinline__ void store_partial(const SplitK &sk, int tile, int split, const v4f (&acc)[4][4]) {
+  v4f *slot = sk.partial + (size_t)(tile * sk.splits + split) * (16 * kQ8Threads) + threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      slot[(i * 4 + j) * kQ8Threads] = acc[i][j];
+}
+
+// The second kernel of a split launch whose kernel wrote partial tiles: thread by thread over every tile's partial
+// sums. A thread takes one accumulator pair, tiles j and j + J/2 of row tile i of one lane of the block layout (the
+// SWIGLU pair, or two plain column tiles), adds the splits in order and applies the epilogue to its four rows. Partial
+// tile layout: [tile][split][i * J + j][THREADS] v4f.
 struct SplitOut {
   Q8Grid grid;
   const v4f *partial;
@@ -749,8 +766,8 @@ __device__ __forceinline__ unsigned short to_bf16(float x) {
 //         feeds value s to the s-th instruction. W rows are read like A rows (row pitch ldw).
 // The FP32 sums stay in the MFMA accumulators: no per-step vector work.
 //
-// Short grids split K; this kernel's register budget leaves room to add the partial tiles in the last block to
-// arrive (split_combine) instead of a second kernel.
+// Short grids split K; this kernel's register budget leaves room to add two or three partial tiles in the last block
+// to arrive (split_combine) instead of a second kernel.
 __global__ __launch_bounds__(256) void bf16_panel(const float *__restrict__ a, long long lda, int m, int k, int kp,
                                                   unsigned short *__restrict__ panel) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x; // 8 values per thread
@@ -925,6 +942,10 @@ template <bool F32> __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds
     advance(step + 4, std::integral_constant<int, 4>{});
   }
   __builtin_amdgcn_s_waitcnt(0);
+  if (p.sk.splits > kCombineSplits) {
+    store_partial(p.sk, tile, split, acc);
+    return;
+  }
   if (p.sk.splits > 1 && !split_combine<kQ8Threads>(p.sk, tile, split, acc))
     return;
   store_tile(seg, t, acc, wm, wn, lane, p.m);
@@ -1111,6 +1132,10 @@ __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_f32x3(MmParams p) {
     advance(step + 5, std::integral_constant<int, 5>{});
   }
   __builtin_amdgcn_s_waitcnt(0);
+  if (p.sk.splits > kCombineSplits) {
+    store_partial(p.sk, tile, split, acc);
+    return;
+  }
   if (p.sk.splits > 1 && !split_combine<kQ8Threads>(p.sk, tile, split, acc))
     return;
   store_tile(seg, t, acc, wm, wn, lane, p.m);
@@ -2246,6 +2271,12 @@ bool f32_on_bf16_parts() {
   return !form || strcmp(form, "fp32") != 0;
 }
 
+// The partial tiles of a split FP32 / BF16 launch added up, where its blocks did not do that themselves.
+bool mm_reduce(const MmParams &p, hipStream_t stream) {
+  return p.sk.splits <= kCombineSplits ||
+         launch_split_reduce<4, kQ8Threads>(p.grid, p.sk, p.m, kQ8TileM, kQ8TileN, stream);
+}
+
 bool x3_launch(MmParams p, hipStream_t stream) {
   static const hipError_t status =
       hipFuncSetAttribute((const void *)mm_gemm_f32x3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kX3Lds);
@@ -2257,7 +2288,7 @@ bool x3_launch(MmParams p, hipStream_t stream) {
   p.sk.partial = (v4f *)device().split_partial;
   p.sk.count = device().split_count;
   hipLaunchKernelGGL(mm_gemm_f32x3, dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), kX3Lds, stream, p);
-  return launch_ok("mm_gemm_f32x3");
+  return launch_ok("mm_gemm_f32x3") && mm_reduce(p, stream);
 }
 
 template <bool F32> bool mm_launch(MmParams p, hipStream_t stream) {
@@ -2272,7 +2303,7 @@ template <bool F32> bool mm_launch(MmParams p, hipStream_t stream) {
   p.sk.count = device().split_count;
   hipLaunchKernelGGL(mm_gemm_lds<F32>, dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), kMmLds, stream,
                      p);
-  return launch_ok(F32 ? "mm_gemm_lds<fp32>" : "mm_gemm_lds<bf16>");
+  return launch_ok(F32 ? "mm_gemm_lds<fp32>" : "mm_gemm_lds<bf16>") && mm_reduce(p, stream);
 }
 
 // The wide BF16 kernel (256 x 256 tiles); its partial tiles are twice the size, so half as many fit the workspace.
