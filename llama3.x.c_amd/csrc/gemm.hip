@@ -4,7 +4,9 @@
 // ADD and SWIGLU (a column tile then holds columns of W1 and the same columns of W3, so the gate is applied in
 // registers). The kernels, each described where it is defined:
 //   q8_gemm_lds     int8, 256 x 128 tiles (or 128 x 128), A/B/scales streamed into LDS five stages deep;
-//   mm_gemm_lds     FP32 and BF16, 256 x 128 tiles, the same pipeline;
+//   mm_gemm_lds     FP32, 256 x 128 tiles, the same pipeline;
+//   mm_gemm_f32x3   FP32 on the BF16 matrix cores, the default FP32 kernel;
+//   bf16_gemm_lds   BF16, 256 x 128 tiles, two K steps a stage;
 //   bf16_gemm_wide  BF16, 256 x 256 tiles for large grids;
 //   split_reduce    the second kernel of a split-K launch of the int8 and wide kernels;
 //   f32_gemm_mfma   FP32 shapes the pipeline does not take (K % 16 != 0, unaligned rows): 128 x 128 tiles staged
@@ -751,22 +753,25 @@ __device__ __forceinline__ unsigned short to_bf16(float x) {
   return (unsigned short)(u >> 16);
 }
 
-// ---- FP32 and BF16: the pipelined MFMA kernel, with split K for short grids ---------------------------------------------
+// ---- FP32 and BF16: the pipelined MFMA kernels, with split K for short grids --------------------------------------------
 //
 // k_gemm_bf16 rounds A to BF16 once per call into the caller's panel (the reference's bf16_convert_rows,
-// src/gemm.c:693-706): rows of kp = K rounded up to 32 values, zero past K. Both modes then share the structure of the
-// int8 kernel above: a 256 x 128 output tile over eight waves of 64 x 64, 4 x 4 MFMA tiles of 16 x 16 per wave, and a
-// K step of 64 bytes per row (32 BF16 or 16 FP32 values) whose A and B tiles go straight from global memory into LDS
-// five stages deep, in 1 KB blocks of 16 rows interleaved by stage. A block row is XOR-swizzled in 16-byte chunks like
-// the int8 tiles. MFMA operands take 16 contiguous bytes of a row per lane group q = lane / 16:
+// src/gemm.c:693-706): rows of kp = K rounded up to 32 values, zero past K. All modes share the structure of the int8
+// kernel above: a 256 x 128 output tile over eight waves of 64 x 64, 4 x 4 MFMA tiles of 16 x 16 per wave, and K steps
+// of 64 bytes per row (32 BF16 or 16 FP32 values) whose A and B tiles go straight from global memory into LDS several
+// steps deep. A block row is XOR-swizzled in 16-byte chunks like the int8 tiles. MFMA operands take 16 contiguous bytes
+// of a row per lane group q = lane / 16:
 //   BF16: v_mfma_f32_16x16x32_bf16, K values 8 q .. 8 q + 7. B arrives in the pack_bf16_vnni layout, whose 16-row
 //         tile and 32-value K step is one contiguous 1 KB block (16 K pairs of 16 rows x 2 values), copied with its
-//         16-byte chunks reordered so that a lane's four K pairs are four conflict-free 4-byte reads.
+//         16-byte chunks reordered so that a lane's four K pairs are four conflict-free 4-byte reads: the block holds
+//         16-byte chunks of one K pair for four rows (chunk 4 P + rg: pair P, rows 4 rg .. 4 rg + 3), and lane l copies
+//         chunk (pair 4 q + p, rows 4 rg ..) with p = l / 16, q = (l / 4) % 4, rg = l % 4 to LDS position
+//         l = 16 p + 4 q + rg, so the MFMA lane (row r, group q) finds its pair 4 q + p at byte 256 p + 64 q + 4 r.
 //   FP32: four v_mfma_f32_16x16x4_f32 per tile and step; lane group q holds K values 4 q .. 4 q + 3 of A and W and
 //         feeds value s to the s-th instruction. W rows are read like A rows (row pitch ldw).
 // The FP32 sums stay in the MFMA accumulators: no per-step vector work.
 //
-// Short grids split K; this kernel's register budget leaves room to add two or three partial tiles in the last block
+// Short grids split K; these kernels' register budgets leave room to add two or three partial tiles in the last block
 // to arrive (split_combine) instead of a second kernel.
 __global__ __launch_bounds__(256) void bf16_panel(const float *__restrict__ a, long long lda, int m, int k, int kp,
                                                   unsigned short *__restrict__ panel) {
@@ -807,7 +812,7 @@ struct MmParams {
   SplitK sk;
 };
 
-template <bool F32> __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds(MmParams p) {
+__global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds(MmParams p) {
   extern __shared__ __align__(16) unsigned char q8_smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -824,23 +829,13 @@ template <bool F32> __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds
   const __amdgpu_buffer_rsrc_t rA = q8_buffer(p.a + (long long)t.m0 * p.arow, (long long)min(kQ8TileM, p.m - t.m0) * p.arow);
   const int offA0 = (int)(ra * p.arow) + ((chunk ^ q8_swizzle(ra)) << 4);
   const int offA1 = (int)((ra + 16) * p.arow) + ((chunk ^ q8_swizzle(ra + 16)) << 4);
-  // B: this wave's 16 rows of one matrix. BF16: one VNNI tile, step s at bytes [s * 1024, s * 1024 + 1024); FP32: 16
-  // weight rows, read like the A rows.
+  // B: this wave's 16 rows of one matrix, read like the A rows
   const int rb0 = 16 * wave;
   const int colB = t.swiglu ? t.n0 + (rb0 & 63) : t.n0 + rb0;
   const unsigned char *wmat = (const unsigned char *)((t.swiglu && rb0 >= 64) ? seg.w3 : seg.w);
-  const long long brow = F32 ? seg.ldw * 4 : 0;
-  const long long tile_bytes = (long long)p.steps * 1024;
-  const __amdgpu_buffer_rsrc_t rB =
-      F32 ? q8_buffer(wmat + (long long)colB * brow, (long long)min(16, seg.n - colB) * brow)
-          : q8_buffer(wmat + (long long)(colB / 16) * tile_bytes, colB < seg.n ? tile_bytes : 0);
-  // BF16: the 1 KB VNNI block holds 16-byte chunks of one K pair for four rows (chunk 4 P + rg: pair P, rows
-  // 4 rg .. 4 rg + 3). Lane l copies chunk (pair 4 q + p, rows 4 rg ..) with p = l / 16, q = (l / 4) % 4, rg = l % 4
-  // to LDS position l = 16 p + 4 q + rg, so the MFMA lane (row r, group q) finds its pair 4 q + p at byte
-  // 256 p + 64 q + 4 r: one 4-byte read per p, on 64 distinct banks across the wave.
-  const int offB = F32 ? (int)(lrow4 * brow) + ((chunk ^ q8_swizzle(lrow4)) << 4)
-                       : ((4 * ((lane >> 2) & 3) + (lane >> 4)) << 6) + ((lane & 3) << 4);
-  const int bstep = F32 ? 64 : 1024; // B bytes per K step
+  const long long brow = seg.ldw * 4;
+  const __amdgpu_buffer_rsrc_t rB = q8_buffer(wmat + (long long)colB * brow, (long long)min(16, seg.n - colB) * brow);
+  const int offB = (int)(lrow4 * brow) + ((chunk ^ q8_swizzle(lrow4)) << 4);
   const __amdgpu_buffer_rsrc_t none = q8_buffer(p.a, 0);
 
   auto issue = [&](int step, auto ST) {
@@ -853,7 +848,7 @@ template <bool F32> __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds
                                              step * 64, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rB : none,
                                              (void *)(q8_smem + kQ8BOff + (wave * kQ8Stages + st) * 1024), 16, offB,
-                                             step * bstep, 0, 0);
+                                             step * 64, 0, 0);
   };
 
   const int lrow = lane & 15, lq = lane >> 4;
@@ -862,8 +857,7 @@ template <bool F32> __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds
   const unsigned char *bbase[4];
 #pragma unroll
   for (int j = 0; j < 4; j++)
-    bbase[j] = q8_smem + kQ8BOff + (b_row(t.swiglu, wn, j) / 16) * kQ8Stages * 1024 +
-               (F32 ? lane_part : lq * 64 + lrow * 4);
+    bbase[j] = q8_smem + kQ8BOff + (b_row(t.swiglu, wn, j) / 16) * kQ8Stages * 1024 + lane_part;
 
   v4f acc[4][4];
 #pragma unroll
@@ -873,40 +867,26 @@ template <bool F32> __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds
       acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
   // MFMA operands of one step, read from LDS a step ahead of their use
-  typedef unsigned v4u __attribute__((ext_vector_type(4)));
   struct Operands {
-    v4u a[4], b[4];
+    v4f a[4], b[4];
   };
   auto operands = [&](auto ST, Operands &o) {
     constexpr int st = decltype(ST)::value;
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      o.a[i] = *reinterpret_cast<const v4u *>(abase + (i * kQ8Stages + st) * 1024);
+      o.a[i] = *reinterpret_cast<const v4f *>(abase + (i * kQ8Stages + st) * 1024);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const unsigned char *bp = bbase[j] + st * 1024;
-      if constexpr (F32)
-        o.b[j] = *reinterpret_cast<const v4u *>(bp);
-      else
-        o.b[j] = v4u{*reinterpret_cast<const unsigned *>(bp), *reinterpret_cast<const unsigned *>(bp + 256),
-                     *reinterpret_cast<const unsigned *>(bp + 512), *reinterpret_cast<const unsigned *>(bp + 768)};
-    }
+    for (int j = 0; j < 4; j++)
+      o.b[j] = *reinterpret_cast<const v4f *>(bbase[j] + st * 1024);
   };
   auto mfmas = [&](const Operands &o) {
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        if constexpr (F32) {
-          const v4f a = __builtin_bit_cast(v4f, o.a[i]), b = __builtin_bit_cast(v4f, o.b[j]);
+      for (int j = 0; j < 4; j++)
 #pragma unroll
-          for (int s = 0; s < 4; s++)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc[i][j], 0, 0, 0);
-        } else {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, o.a[i]),
-                                                              __builtin_bit_cast(v8bf_t, o.b[j]), acc[i][j], 0, 0, 0);
-        }
-      }
+        for (int s = 0; s < 4; s++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[i][s], o.b[j][s], acc[i][j], 0, 0, 0);
   };
 
   // One step in stage ST: step + 1's loads have landed once only the two later steps' may be outstanding; the barrier
@@ -940,6 +920,157 @@ template <bool F32> __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds
     advance(step + 2, std::integral_constant<int, 2>{});
     advance(step + 3, std::integral_constant<int, 3>{});
     advance(step + 4, std::integral_constant<int, 4>{});
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  if (p.sk.splits > kCombineSplits) {
+    store_partial(p.sk, tile, split, acc);
+    return;
+  }
+  if (p.sk.splits > 1 && !split_combine<kQ8Threads>(p.sk, tile, split, acc))
+    return;
+  store_tile(seg, t, acc, wm, wn, lane, p.m);
+}
+
+// ---- BF16, 256 x 128 tiles ----------------------------------------------------------------------------------------
+//
+// Delivery of the operands bounds the BF16 tiles, not the MFMAs (a copy of a kernel with 64-byte steps and five stages
+// took the same time without its MFMAs): a row's 64 bytes of A are half a cache line, so each step fetched the line of
+// the step before again. Here a stage takes two steps, 128 bytes of each row, as eight rows per 1 KB load; three stages
+// of 48 KB hold as many steps in flight. A row's eight 16-byte chunks lie at chunk ^ (row % 8), so the operand reads of
+// eight consecutive rows fall on distinct banks. Measured, 64-byte steps / this (us, the panel's rounding included): 512
+// x 2 * 8192 x 3072 SwiGLU 71 / 58 (880 TFLOP/s), 512 x 3072 x 8192 56 / 50, 512 x 5120 x 3072 41 / 37, 2048 x 3072 x
+// 8192 195 / 158 (650 TFLOP/s). Without its loads the SwiGLU shape takes 50: LDS reads and MFMAs, 1.2 PFLOP/s, the rate
+// a library product of 8192 cubed reaches here.
+constexpr int kBfStages = 3, kBfLoads = 6;                       // per wave and pair of steps: four A and two B blocks
+constexpr int kBfBOff = (kQ8TileM / 8) * kBfStages * 1024;        // A: 32 blocks of 8 rows a stage
+constexpr size_t kBfLds = (size_t)kBfBOff + 2 * kQ8BBlocks * kBfStages * 1024; // 144 KB
+static_assert(kBfLds <= 160 * 1024, "one BF16 block fits a CU's LDS");
+
+__global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_lds(MmParams p) {
+  extern __shared__ __align__(16) unsigned char q8_smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int logical = xcd_logical(blockIdx.x, p.grid.total * p.sk.splits);
+  const int tile = __builtin_amdgcn_readfirstlane(logical / p.sk.splits); // uniform (see q8_gemm_lds)
+  const int split = __builtin_amdgcn_readfirstlane(logical % p.sk.splits);
+  const TilePos t = q8_tile_of(p.grid, tile);
+  const TileSeg seg = q8_seg_of(p.grid, t.s);
+  const int s0 = split * p.sk.per, s1 = min(p.steps, s0 + p.sk.per); // s0 is even
+
+  // A block i of the wave: rows 32 wave + 8 i .., lane l row l / 8, its 16 bytes chunk (l % 8) ^ (l / 8) of the pair's
+  // 128. The second step of a pair past s1 reads zeros (an offset past the buffer): its chunks hold the next row's
+  // values, or the next split's.
+  const int arow8 = lane >> 3, achunk = (lane & 7) ^ arow8;
+  const __amdgpu_buffer_rsrc_t rA = q8_buffer(p.a + (long long)t.m0 * p.arow, (long long)min(kQ8TileM, p.m - t.m0) * p.arow);
+  int offA[4]; // per block: the bounds check that makes rows past m read zeros sees the lane's offset alone
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    offA[i] = (int)((32 * wave + 8 * i + arow8) * p.arow) + (achunk << 4);
+  // B: the wave's column tile, one VNNI tile of one matrix, two 1 KB steps of it (chunks reordered as described above)
+  const int rb0 = 16 * wave;
+  const int colB = t.swiglu ? t.n0 + (rb0 & 63) : t.n0 + rb0;
+  const unsigned char *wmat = (const unsigned char *)((t.swiglu && rb0 >= 64) ? seg.w3 : seg.w);
+  const long long tile_bytes = (long long)p.steps * 1024;
+  const __amdgpu_buffer_rsrc_t rB =
+      q8_buffer(wmat + (long long)(colB / 16) * tile_bytes, colB < seg.n ? tile_bytes : 0);
+  const int offB = ((4 * ((lane >> 2) & 3) + (lane >> 4)) << 6) + ((lane & 3) << 4);
+  const __amdgpu_buffer_rsrc_t none = q8_buffer(p.a, 0);
+
+  // steps `step` (even) and step + 1 into stage ST
+  auto issue = [&](int step, auto ST) {
+    constexpr int st = decltype(ST)::value;
+    const bool live = step < s1, both = step + 1 < s1;
+    const bool past = !both && achunk >= 4;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rA : none,
+                                               (void *)(q8_smem + ((4 * wave + i) * kBfStages + st) * 1024), 16,
+                                               past ? 0x7FFFFF00 : offA[i], step * 64, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rB : none,
+                                             (void *)(q8_smem + kBfBOff + (2 * wave * kBfStages + st) * 1024), 16, offB,
+                                             step * 1024, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(both ? rB : none,
+                                             (void *)(q8_smem + kBfBOff + ((2 * wave + 1) * kBfStages + st) * 1024), 16,
+                                             offB, step * 1024 + 1024, 0, 0);
+  };
+
+  // Operand reads of step H of a pair: lane (row r = l % 16, group q = l / 16) takes chunk 4 H + q of A's row r, held
+  // at (4 H + q) ^ (r % 8), and K pairs 4 q .. 4 q + 3 of B's row r.
+  const int lrow = lane & 15, lq = lane >> 4;
+  const unsigned char *arow0 = q8_smem + (8 * wm + (lrow >> 3)) * kBfStages * 1024 + (lrow & 7) * 128;
+  const unsigned char *abase[2] = {arow0 + ((lq ^ (lrow & 7)) << 4), arow0 + (((4 + lq) ^ (lrow & 7)) << 4)};
+  const unsigned char *bbase[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    bbase[j] = q8_smem + kBfBOff + (b_row(t.swiglu, wn, j) / 16) * 2 * kBfStages * 1024 + lq * 64 + lrow * 4;
+
+  v4f acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  struct Operands {
+    v4u a[4], b[4];
+  };
+  auto operands = [&](auto ST, auto H, Operands &o) {
+    constexpr int st = decltype(ST)::value, h = decltype(H)::value;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      o.a[i] = *reinterpret_cast<const v4u *>(abase[h] + (2 * i * kBfStages + st) * 1024);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const unsigned char *bp = bbase[j] + (h * kBfStages + st) * 1024;
+      o.b[j] = v4u{*reinterpret_cast<const unsigned *>(bp), *reinterpret_cast<const unsigned *>(bp + 256),
+                   *reinterpret_cast<const unsigned *>(bp + 512), *reinterpret_cast<const unsigned *>(bp + 768)};
+    }
+  };
+  auto mfmas = [&](const Operands &o) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, o.a[i]),
+                                                            __builtin_bit_cast(v8bf_t, o.b[j]), acc[i][j], 0, 0, 0);
+  };
+
+  // The pair in stage ST: its first step's MFMAs (operands already in registers) while the second step's are read;
+  // then every wave is done with the stage once its reads are, the next pair has landed once only the one after it may
+  // be outstanding, and the pair three further fills the stage while the second step's MFMAs run.
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, 1> second{};
+  Operands cur, next;
+  auto advance = [&](int step, auto ST) {
+    constexpr int nst = (decltype(ST)::value + 1) % kBfStages;
+    operands(ST, second, next);
+    __builtin_amdgcn_sched_barrier(0);
+    mfmas(cur);
+    __builtin_amdgcn_sched_barrier(0);
+    cur = next;
+    wait_vmcnt_lgkm0<kBfLoads>();
+    __builtin_amdgcn_s_barrier();
+    issue(step + 2 * kBfStages, ST);
+    operands(std::integral_constant<int, nst>{}, first, next);
+    __builtin_amdgcn_sched_barrier(0);
+    mfmas(cur);
+    __builtin_amdgcn_sched_barrier(0);
+    cur = next;
+  };
+
+  issue(s0, std::integral_constant<int, 0>{});
+  issue(s0 + 2, std::integral_constant<int, 1>{});
+  issue(s0 + 4, std::integral_constant<int, 2>{});
+  wait_vmcnt<(kBfStages - 1) * kBfLoads>();
+  __builtin_amdgcn_s_barrier();
+  operands(std::integral_constant<int, 0>{}, first, cur);
+  // whole rounds of three pairs: pairs past the end load zeros and add nothing (exits inside a round cost the 512 x 2 *
+  // 8192 x 3072 shape 1.5 us)
+  for (int step = s0; step < s1; step += 2 * kBfStages) {
+    advance(step, std::integral_constant<int, 0>{});
+    advance(step + 2, std::integral_constant<int, 1>{});
+    advance(step + 4, std::integral_constant<int, 2>{});
   }
   __builtin_amdgcn_s_waitcnt(0);
   if (p.sk.splits > kCombineSplits) {
@@ -2265,7 +2396,7 @@ bool launch_q8_group_dots(int32_t *dots, const int8_t *xq, int m, int k, int gs,
 namespace {
 
 // Which kernel takes the aligned FP32 GEMM: mm_gemm_f32x3 (products from exact BF16 parts; 3B prefill GEMMs at 512
-// rows 23.7 -> 17.0 ms) unless LLAMA_HIP_F32_FORM = fp32 picks mm_gemm_lds<true> (FP32 products); read on every call.
+// rows 23.7 -> 17.0 ms) unless LLAMA_HIP_F32_FORM = fp32 picks mm_gemm_lds (FP32 products); read on every call.
 bool f32_on_bf16_parts() {
   const char *form = getenv("LLAMA_HIP_F32_FORM");
   return !form || strcmp(form, "fp32") != 0;
@@ -2291,19 +2422,22 @@ bool x3_launch(MmParams p, hipStream_t stream) {
   return launch_ok("mm_gemm_f32x3") && mm_reduce(p, stream);
 }
 
+// The FP32-product kernel, or the BF16 one, whose K loop runs whole rounds of its stages, two steps each: so do its
+// splits (512 x 3072 x 3072: four of 24 steps 31.4 us, five of 20, which run 24 each, 32.9).
 template <bool F32> bool mm_launch(MmParams p, hipStream_t stream) {
+  const auto kernel = F32 ? mm_gemm_lds : bf16_gemm_lds;
+  constexpr size_t lds = F32 ? kMmLds : kBfLds;
   static const hipError_t status =
-      hipFuncSetAttribute((const void *)mm_gemm_lds<F32>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMmLds);
+      hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (!check_hip(status, "allowing the FP32 / BF16 GEMM its LDS"))
     return false;
-  p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, p.steps, &p.sk.per);
+  p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, p.steps, &p.sk.per, F32 ? 1 : 2 * kBfStages);
   if (p.sk.splits == 1)
     p.sk.per = p.steps;
   p.sk.partial = (v4f *)device().split_partial;
   p.sk.count = device().split_count;
-  hipLaunchKernelGGL(mm_gemm_lds<F32>, dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), kMmLds, stream,
-                     p);
-  return launch_ok(F32 ? "mm_gemm_lds<fp32>" : "mm_gemm_lds<bf16>") && mm_reduce(p, stream);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), lds, stream, p);
+  return launch_ok(F32 ? "mm_gemm_lds" : "bf16_gemm_lds") && mm_reduce(p, stream);
 }
 
 // The wide BF16 kernel (256 x 256 tiles); its partial tiles are twice the size, so half as many fit the workspace.

@@ -362,3 +362,36 @@ def test_pipelined_gemm_split_k(m, n, k, mode, monkeypatch):
         L.llhip_set_gemm_splits(0)
         L.llhip_set_bf16_tile(0)
         L.aligned_buffer_free(panel)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (3, 130, 96), (255, 17, 160), (257, 128, 224), (16, 64, 448), (40, 144, 66)])
+def test_bf16_gemm_odd_steps_and_neighbours(m, n, k):
+    """The BF16 kernel's stages hold two 32-value K steps: odd step counts, K ranges of a split that end inside a stage,
+    and rows at the edges of a tile. Every second row of A is infinite, so a finite row that took any of its
+    neighbour's values (which follow its own in memory) would come out infinite or NaN; finite rows stay within
+    2e-6 * sum|a w| of float64 on the BF16 operands (FP32 sums of at most 448 terms, 2^-24 each)."""
+    L = hu.lib()
+    L.llhip_set_bf16_tile(1)
+    rng = orc.Rng(orc.SEED + 97 * m + n + k)
+    a = rng.uniform(m * k, 2.0).reshape(m, k)
+    a[1::2] = np.inf
+    w = rng.uniform(n * k).reshape(n, k)
+    pw = np.zeros(L.bf16_vnni_elements(n, k), np.uint16)
+    L.pack_bf16_vnni(lh.ptr(pw), lh.ptr(w), n, k, k)
+    da, dw = hu.dev(a), hu.dev(pw)
+    r, mag = ref_f32(bf16_round(a[::2].copy()), bf16_round(w))
+    panel = lh.AlignedBuffer()
+    L.aligned_buffer_alloc(panel, L.k_gemm_bf16_panel_bytes(m, k), 1)
+    try:
+        for splits in (0, 1, 2, 4):
+            L.llhip_set_gemm_splits(splits)
+            dc = hu.dev(np.zeros((m, n), np.float32))
+            seg = lh.GemmBf16Segment(lh.ptr(dc), n, lh.ptr(dw), None, n, lh.GEMM_STORE)
+            L.k_gemm_bf16(lh.ptr(da), k, m, k, seg, 1, panel)
+            got = hu.host(dc)
+            hu.assert_within_budget(got[::2], r, mag, rel=2e-6, what=f"{m}x{n}x{k} splits {splits}")
+            assert not np.isfinite(got[1::2]).any()
+    finally:
+        L.llhip_set_gemm_splits(0)
+        L.llhip_set_bf16_tile(0)
+        L.aligned_buffer_free(panel)
