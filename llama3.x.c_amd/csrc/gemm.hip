@@ -96,14 +96,16 @@ __device__ __forceinline__ int b_row(bool swiglu, int wn, int j) {
   return swiglu ? (j < 2 ? 32 * wn + 16 * j : 64 + 32 * wn + 16 * (j - 2)) : 64 * wn + 16 * j;
 }
 
-__device__ __forceinline__ void store_tile(const TileSeg &seg, const TilePos &t, const v4f (&acc)[4][4], int wm, int wn,
+// MI: 16-row MFMA tiles of a wave (its rows start at 16 MI wm).
+template <int MI>
+__device__ __forceinline__ void store_tile(const TileSeg &seg, const TilePos &t, const v4f (&acc)[MI][4], int wm, int wn,
                                            int lane, int m) {
   const int lc = lane & 15, lr = (lane >> 4) * 4;
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int row = t.m0 + wm * 64 + 16 * i + lr + e;
+      const int row = t.m0 + wm * 16 * MI + 16 * i + lr + e;
       if (row >= m)
         continue;
       float *crow = seg.c + (long long)row * seg.ldc;
@@ -385,15 +387,15 @@ constexpr int kCombineSplits = 3;
 constexpr int kDeviceCoherent = 16;
 
 // The last of a tile's blocks to arrive gets true with acc holding the whole sum; the others get false.
-template <int THREADS>
-__device__ __forceinline__ bool split_combine(const SplitK &sk, int tile, int split, v4f (&acc)[4][4]) {
+template <int THREADS, int MI>
+__device__ __forceinline__ bool split_combine(const SplitK &sk, int tile, int split, v4f (&acc)[MI][4]) {
   __shared__ int last;
   const int tid = threadIdx.x;
-  constexpr int kSlotBytes = 16 * THREADS * 16; // one partial tile
+  constexpr int kSlotBytes = 4 * MI * THREADS * 16; // one partial tile
   const __amdgpu_buffer_rsrc_t r =
       q8_buffer((const unsigned char *)sk.partial + (size_t)tile * sk.splits * kSlotBytes, (long long)sk.splits * kSlotBytes);
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++)
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, acc[i][j]), r,
@@ -407,15 +409,15 @@ __device__ __forceinline__ bool split_combine(const SplitK &sk, int tile, int sp
   __syncthreads();
   if (!last)
     return false;
-  v4f own[4][4];
+  v4f own[MI][4];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++)
       own[i][j] = acc[i][j];
   for (int s = 0; s < sk.splits; s++) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < MI; i++)
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const v4f v = s == split ? own[i][j]
@@ -431,10 +433,11 @@ __device__ __forceinline__ bool split_combine(const SplitK &sk, int tile, int sp
 }
 
 // A block's partial tile into its slot, for split_reduce.
-__device__ __forceinline__ void store_partial(const SplitK &sk, int tile, int split, const v4f (&acc)[4][4]) {
-  v4f *slot = sk.partial + (size_t)(tile * sk.splits + split) * (16 * kQ8Threads) + threadIdx.x;
+template <int MI>
+__device__ __forceinline__ void store_partial(const SplitK &sk, int tile, int split, const v4f (&acc)[MI][4]) {
+  v4f *slot = sk.partial + (size_t)(tile * sk.splits + split) * (4 * MI * kQ8Threads) + threadIdx.x;
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++)
       slot[(i * 4 + j) * kQ8Threads] = acc[i][j];
@@ -443,23 +446,23 @@ __device__ __forceinline__ void store_partial(const SplitK &sk, int tile, int sp
 // The second kernel of a split launch whose kernel wrote partial tiles: thread by thread over every tile's partial
 // sums. A thread takes one accumulator pair, tiles j and j + J/2 of row tile i of one lane of the block layout (the
 // SWIGLU pair, or two plain column tiles), adds the splits in order and applies the epilogue to its four rows. Partial
-// tile layout: [tile][split][i * J + j][THREADS] v4f.
+// tile layout: [tile][split][i * J + j][THREADS] v4f, i below MI.
 struct SplitOut {
   Q8Grid grid;
   const v4f *partial;
   int splits, m, tile_m, tile_n;
 };
 
-template <int J, int THREADS> __global__ __launch_bounds__(256) void split_reduce(SplitOut p) {
+template <int J, int THREADS, int MI> __global__ __launch_bounds__(256) void split_reduce(SplitOut p) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long per_tile = 4LL * (J / 2) * THREADS;
+  const long long per_tile = (long long)MI * (J / 2) * THREADS;
   if (idx >= per_tile * p.grid.total)
     return;
   const int tile = (int)(idx / per_tile), rest = (int)(idx % per_tile);
   const int tid = rest % THREADS, jp = (rest / THREADS) % (J / 2), i = rest / THREADS / (J / 2);
   const TilePos t = q8_tile_of(p.grid, tile, p.tile_m, p.tile_n);
   const TileSeg seg = q8_seg_of(p.grid, t.s);
-  const v4f *part = p.partial + (size_t)tile * p.splits * (4 * J * THREADS) + tid;
+  const v4f *part = p.partial + (size_t)tile * p.splits * (MI * J * THREADS) + tid;
   // The partials are added in split order; they are loaded kBatch splits at a time, all in flight together (a loop
   // that adds each as it arrives waits for one load per split). Past the last split a load repeats the last one and
   // its sum is not taken.
@@ -470,7 +473,7 @@ template <int J, int THREADS> __global__ __launch_bounds__(256) void split_reduc
     v4f l[kBatch], h[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; u++) {
-      const size_t at = (size_t)min(s0 + u, p.splits - 1) * (4 * J * THREADS);
+      const size_t at = (size_t)min(s0 + u, p.splits - 1) * (MI * J * THREADS);
       l[u] = part[at + lo_at];
       h[u] = part[at + hi_at];
     }
@@ -488,18 +491,18 @@ template <int J, int THREADS> __global__ __launch_bounds__(256) void split_reduc
   const int lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
   const int lc = lane & 15, lr = (lane >> 4) * 4;
   constexpr int kSpan = 16 * J; // columns a wave covers
-  const int rows = min(4, p.m - (t.m0 + wm * 64 + 16 * i + lr)); // this thread's rows below m
+  const int rows = min(4, p.m - (t.m0 + wm * 16 * MI + 16 * i + lr)); // this thread's rows below m
   if (t.swiglu) {
     const int col = t.n0 + (kSpan / 2) * wn + 16 * jp + lc;
 #pragma unroll
     for (int e = 0; e < 4; e++)
       if (e < rows && col < seg.n)
-        seg.c[(long long)(t.m0 + wm * 64 + 16 * i + lr + e) * seg.ldc + col] = silu_gate(lo[e], hi[e]);
+        seg.c[(long long)(t.m0 + wm * 16 * MI + 16 * i + lr + e) * seg.ldc + col] = silu_gate(lo[e], hi[e]);
     return;
   }
   const int c0 = t.n0 + kSpan * wn + 16 * jp + lc, c1 = c0 + 16 * (J / 2);
   const bool in0 = c0 < seg.n, in1 = c1 < seg.n;
-  float *crow0 = seg.c + (long long)(t.m0 + wm * 64 + 16 * i + lr) * seg.ldc;
+  float *crow0 = seg.c + (long long)(t.m0 + wm * 16 * MI + 16 * i + lr) * seg.ldc;
   if (seg.epi == EPI_ADD) { // every current value read before any sum is written back
     float prior0[4], prior1[4];
 #pragma unroll
@@ -538,6 +541,25 @@ template <int I, int N, class F> __device__ __forceinline__ void issue_first(F &
   if constexpr (I < N) {
     f(first + I, std::integral_constant<int, I>{});
     issue_first<I + 1, N>(f, first);
+  }
+}
+
+// A round of N stages of two K steps, leaving after the last pair when EXITS (then false).
+template <int I, int N, bool EXITS, class F> __device__ __forceinline__ bool pair_round(F &f, int step, int steps) {
+  if constexpr (I < N) {
+    f(step + 2 * I, std::integral_constant<int, I>{});
+    if (EXITS && I + 1 < N && step + 2 * I + 2 >= steps)
+      return false;
+    return pair_round<I + 1, N, EXITS>(f, step, steps);
+  }
+  return true;
+}
+
+// The loads of the first N pairs of steps into stages 0 .. N - 1.
+template <int I, int N, class F> __device__ __forceinline__ void issue_first_pairs(F &f, int first) {
+  if constexpr (I < N) {
+    f(first + 2 * I, std::integral_constant<int, I>{});
+    issue_first_pairs<I + 1, N>(f, first);
   }
 }
 
@@ -941,12 +963,22 @@ __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds(MmParams p) {
 // x 2 * 8192 x 3072 SwiGLU 71 / 58 (880 TFLOP/s), 512 x 3072 x 8192 56 / 50, 512 x 5120 x 3072 41 / 37, 2048 x 3072 x
 // 8192 195 / 158 (650 TFLOP/s). Without its loads the SwiGLU shape takes 50: LDS reads and MFMAs, 1.2 PFLOP/s, the rate
 // a library product of 8192 cubed reaches here.
-constexpr int kBfStages = 3, kBfLoads = 6;                       // per wave and pair of steps: four A and two B blocks
-constexpr int kBfBOff = (kQ8TileM / 8) * kBfStages * 1024;        // A: 32 blocks of 8 rows a stage
-constexpr size_t kBfLds = (size_t)kBfBOff + 2 * kQ8BBlocks * kBfStages * 1024; // 144 KB
-static_assert(kBfLds <= 160 * 1024, "one BF16 block fits a CU's LDS");
+// The same tile and stage shapes serve the FP32 form on BF16 parts (a stage holds 32 FP32 values of each row). MI is
+// the wave's 16-row MFMA tiles: 256, 192, 128 or 64 rows a block, the fewest that hold the batch in as many row tiles
+// as 256-row blocks take, with more stages where the rows are few and the weights' latency is what there is to hide
+// (BF16, 256-row tiles / this: 20 x 2 * 8192 x 2048 31 / 21 us, 20 x 2048 x 8192 26 / 19, 180 x 4096 x 4096 28 / 26, 300
+// x 4096 x 14336 74 / 64).
+template <int MI_, int STAGES_> struct MmCfg {
+  static constexpr int MI = MI_, Stages = STAGES_, TileM = 64 * MI;
+  static constexpr int Loads = MI + 2;                        // per wave and stage: MI blocks of A and two of B
+  static constexpr int BOff = 8 * MI * Stages * 1024;          // A: 8 MI blocks of 8 rows a stage, then 16 blocks of B
+  static constexpr size_t Lds = (size_t)BOff + 16 * Stages * 1024;
+  static_assert(Lds < 160 * 1024, "a block and split_combine's flag fit a CU's LDS");
+};
+template <int MI> using MmTile = MmCfg<MI, MI == 1 ? 6 : MI == 2 ? 4 : 3>;
 
-__global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_lds(MmParams p) {
+template <class C> __global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_lds(MmParams p) {
+  constexpr int MI = C::MI;
   extern __shared__ __align__(16) unsigned char q8_smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -954,19 +986,19 @@ __global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_lds(MmParams p) {
   const int logical = xcd_logical(blockIdx.x, p.grid.total * p.sk.splits);
   const int tile = __builtin_amdgcn_readfirstlane(logical / p.sk.splits); // uniform (see q8_gemm_lds)
   const int split = __builtin_amdgcn_readfirstlane(logical % p.sk.splits);
-  const TilePos t = q8_tile_of(p.grid, tile);
+  const TilePos t = q8_tile_of(p.grid, tile, C::TileM);
   const TileSeg seg = q8_seg_of(p.grid, t.s);
   const int s0 = split * p.sk.per, s1 = min(p.steps, s0 + p.sk.per); // s0 is even
 
-  // A block i of the wave: rows 32 wave + 8 i .., lane l row l / 8, its 16 bytes chunk (l % 8) ^ (l / 8) of the pair's
+  // A block i of the wave: rows 8 (MI wave + i) .., lane l row l / 8, its 16 bytes chunk (l % 8) ^ (l / 8) of the pair's
   // 128. The second step of a pair past s1 reads zeros (an offset past the buffer): its chunks hold the next row's
   // values, or the next split's.
   const int arow8 = lane >> 3, achunk = (lane & 7) ^ arow8;
-  const __amdgpu_buffer_rsrc_t rA = q8_buffer(p.a + (long long)t.m0 * p.arow, (long long)min(kQ8TileM, p.m - t.m0) * p.arow);
-  int offA[4]; // per block: the bounds check that makes rows past m read zeros sees the lane's offset alone
+  const __amdgpu_buffer_rsrc_t rA = q8_buffer(p.a + (long long)t.m0 * p.arow, (long long)min(C::TileM, p.m - t.m0) * p.arow);
+  int offA[4]; // per block (MI used): the bounds check that makes rows past m read zeros sees the lane's offset alone
 #pragma unroll
-  for (int i = 0; i < 4; i++)
-    offA[i] = (int)((32 * wave + 8 * i + arow8) * p.arow) + (achunk << 4);
+  for (int i = 0; i < MI; i++)
+    offA[i] = (int)((8 * (MI * wave + i) + arow8) * p.arow) + (achunk << 4);
   // B: the wave's column tile, one VNNI tile of one matrix, two 1 KB steps of it (chunks reordered as described above)
   const int rb0 = 16 * wave;
   const int colB = t.swiglu ? t.n0 + (rb0 & 63) : t.n0 + rb0;
@@ -983,53 +1015,53 @@ __global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_lds(MmParams p) {
     const bool live = step < s1, both = step + 1 < s1;
     const bool past = !both && achunk >= 4;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < MI; i++)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rA : none,
-                                               (void *)(q8_smem + ((4 * wave + i) * kBfStages + st) * 1024), 16,
-                                               past ? 0x7FFFFF00 : offA[i], step * 64, 0, 0);
+                                               (void *)(q8_smem + ((MI * wave + i) * C::Stages + st) * 1024), 16,
+                                               past ? 0x7FFFFFF0 : offA[i], step * 64, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rB : none,
-                                             (void *)(q8_smem + kBfBOff + (2 * wave * kBfStages + st) * 1024), 16, offB,
+                                             (void *)(q8_smem + C::BOff + (2 * wave * C::Stages + st) * 1024), 16, offB,
                                              step * 1024, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(both ? rB : none,
-                                             (void *)(q8_smem + kBfBOff + ((2 * wave + 1) * kBfStages + st) * 1024), 16,
+                                             (void *)(q8_smem + C::BOff + ((2 * wave + 1) * C::Stages + st) * 1024), 16,
                                              offB, step * 1024 + 1024, 0, 0);
   };
 
   // Operand reads of step H of a pair: lane (row r = l % 16, group q = l / 16) takes chunk 4 H + q of A's row r, held
   // at (4 H + q) ^ (r % 8), and K pairs 4 q .. 4 q + 3 of B's row r.
   const int lrow = lane & 15, lq = lane >> 4;
-  const unsigned char *arow0 = q8_smem + (8 * wm + (lrow >> 3)) * kBfStages * 1024 + (lrow & 7) * 128;
+  const unsigned char *arow0 = q8_smem + (2 * MI * wm + (lrow >> 3)) * C::Stages * 1024 + (lrow & 7) * 128;
   const unsigned char *abase[2] = {arow0 + ((lq ^ (lrow & 7)) << 4), arow0 + (((4 + lq) ^ (lrow & 7)) << 4)};
   const unsigned char *bbase[4];
 #pragma unroll
   for (int j = 0; j < 4; j++)
-    bbase[j] = q8_smem + kBfBOff + (b_row(t.swiglu, wn, j) / 16) * 2 * kBfStages * 1024 + lq * 64 + lrow * 4;
+    bbase[j] = q8_smem + C::BOff + (b_row(t.swiglu, wn, j) / 16) * 2 * C::Stages * 1024 + lq * 64 + lrow * 4;
 
-  v4f acc[4][4];
+  v4f acc[MI][4];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++)
       acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   typedef unsigned v4u __attribute__((ext_vector_type(4)));
   struct Operands {
-    v4u a[4], b[4];
+    v4u a[MI], b[4];
   };
   auto operands = [&](auto ST, auto H, Operands &o) {
     constexpr int st = decltype(ST)::value, h = decltype(H)::value;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-      o.a[i] = *reinterpret_cast<const v4u *>(abase[h] + (2 * i * kBfStages + st) * 1024);
+    for (int i = 0; i < MI; i++)
+      o.a[i] = *reinterpret_cast<const v4u *>(abase[h] + (2 * i * C::Stages + st) * 1024);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      const unsigned char *bp = bbase[j] + (h * kBfStages + st) * 1024;
+      const unsigned char *bp = bbase[j] + (h * C::Stages + st) * 1024;
       o.b[j] = v4u{*reinterpret_cast<const unsigned *>(bp), *reinterpret_cast<const unsigned *>(bp + 256),
                    *reinterpret_cast<const unsigned *>(bp + 512), *reinterpret_cast<const unsigned *>(bp + 768)};
     }
   };
   auto mfmas = [&](const Operands &o) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < MI; i++)
 #pragma unroll
       for (int j = 0; j < 4; j++)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, o.a[i]),
@@ -1037,21 +1069,21 @@ __global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_lds(MmParams p) {
   };
 
   // The pair in stage ST: its first step's MFMAs (operands already in registers) while the second step's are read;
-  // then every wave is done with the stage once its reads are, the next pair has landed once only the one after it may
-  // be outstanding, and the pair three further fills the stage while the second step's MFMAs run.
+  // then every wave is done with the stage once its reads are, the next pair has landed once only those after it may be
+  // outstanding, and the pair Stages further fills the stage while the second step's MFMAs run.
   constexpr std::integral_constant<int, 0> first{};
   constexpr std::integral_constant<int, 1> second{};
   Operands cur, next;
   auto advance = [&](int step, auto ST) {
-    constexpr int nst = (decltype(ST)::value + 1) % kBfStages;
+    constexpr int nst = (decltype(ST)::value + 1) % C::Stages;
     operands(ST, second, next);
     __builtin_amdgcn_sched_barrier(0);
     mfmas(cur);
     __builtin_amdgcn_sched_barrier(0);
     cur = next;
-    wait_vmcnt_lgkm0<kBfLoads>();
+    wait_vmcnt_lgkm0<(C::Stages - 2) * C::Loads>();
     __builtin_amdgcn_s_barrier();
-    issue(step + 2 * kBfStages, ST);
+    issue(step + 2 * C::Stages, ST);
     operands(std::integral_constant<int, nst>{}, first, next);
     __builtin_amdgcn_sched_barrier(0);
     mfmas(cur);
@@ -1059,19 +1091,15 @@ __global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_lds(MmParams p) {
     cur = next;
   };
 
-  issue(s0, std::integral_constant<int, 0>{});
-  issue(s0 + 2, std::integral_constant<int, 1>{});
-  issue(s0 + 4, std::integral_constant<int, 2>{});
-  wait_vmcnt<(kBfStages - 1) * kBfLoads>();
+  issue_first_pairs<0, C::Stages>(issue, s0);
+  wait_vmcnt<(C::Stages - 1) * C::Loads>();
   __builtin_amdgcn_s_barrier();
   operands(std::integral_constant<int, 0>{}, first, cur);
-  // whole rounds of three pairs: pairs past the end load zeros and add nothing (exits inside a round cost the 512 x 2 *
-  // 8192 x 3072 shape 1.5 us)
-  for (int step = s0; step < s1; step += 2 * kBfStages) {
-    advance(step, std::integral_constant<int, 0>{});
-    advance(step + 2, std::integral_constant<int, 1>{});
-    advance(step + 4, std::integral_constant<int, 2>{});
-  }
+  // Whole rounds of stages where the sums fill the registers: pairs past the end load zeros and add nothing (exits inside
+  // a round cost the 512 x 2 * 8192 x 3072 shape 1.5 us). Fewer rows leave a round after the last pair.
+  for (int step = s0; step < s1; step += 2 * C::Stages)
+    if (!pair_round<0, C::Stages, (MI <= 2)>(advance, step, s1))
+      break;
   __builtin_amdgcn_s_waitcnt(0);
   if (p.sk.splits > kCombineSplits) {
     store_partial(p.sk, tile, split, acc);
@@ -1088,16 +1116,15 @@ __global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_lds(MmParams p) {
 // the batched attention forms them: x = h + m + l exactly (h the top 8 significant bits of x, m the next 8 of x - h, l
 // the rest, at most 8 bits) and x y is taken as hh + hm + mh + mm + hl + lh, the dropped products below 2^-23 of |x y|
 // and every BF16 product exact in FP32, so each sum is FP32-accurate. Six v_mfma_f32_16x16x32_bf16 (16 cycles) replace
-// eight v_mfma_f32_16x16x4_f32 (32 cycles each). The tiles, A and W staging (64 bytes of 16 rows per 1 KB block, XOR
-// swizzle, buffer loads straight into LDS), split K and epilogues are mm_gemm_lds's FP32 ones, with six stages so
-// that a round of steps is a whole number of pairs: the MFMAs run at every second step on the K values of the pair,
-// lane group q's slots 8 q .. 8 q + 3 from the first step's values 4 q .. 4 q + 3 and slots 8 q + 4 .. from the
-// second's, the same in A and in W, and each lane splits its own operands in registers.
-constexpr int kX3Stages = 6;
-constexpr int kX3BOff = kQ8ABlocks * kX3Stages * 1024;
-constexpr size_t kX3Lds = (size_t)kX3BOff + (size_t)kQ8BBlocks * kX3Stages * 1024;
-
-__global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_f32x3(MmParams p) {
+// eight v_mfma_f32_16x16x4_f32 (32 cycles each). The tiles and stages are bf16_gemm_lds's: a stage holds two K steps of
+// 16 values, 128 bytes of each row of A and of W, and the MFMAs run once per stage, lane group q's slots 8 q .. 8 q + 3
+// from the first step's values 4 q .. 4 q + 3 and slots 8 q + 4 .. from the second's, the same in A and in W; each lane
+// splits its own operands in registers. The MFMAs bound it (at 512 rows the W1/W3 product runs at the rate of a large
+// BF16 product), so the rows a tile holds past the batch cost in full. Measured,
+// 256-row tiles and 64-byte stages / this (us): 333 x 2 * 8192 x 3072 SwiGLU 242 / 202, 333 x 3072 x 8192 156 / 118 (142
+// TFLOP/s of FP32 products), 512 x 2 * 8192 x 3072 273 / 260, 20 x 2 * 8192 x 2048 87 / 42, 64 x 3072 x 3072 43 / 22.
+template <class C> __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_f32x3(MmParams p) {
+  constexpr int MI = C::MI;
   extern __shared__ __align__(16) unsigned char q8_smem[];
   typedef int v4i_t __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63;
@@ -1106,62 +1133,71 @@ __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_f32x3(MmParams p) {
   const int logical = xcd_logical(blockIdx.x, p.grid.total * p.sk.splits);
   const int tile = __builtin_amdgcn_readfirstlane(logical / p.sk.splits);
   const int split = __builtin_amdgcn_readfirstlane(logical % p.sk.splits);
-  const TilePos t = q8_tile_of(p.grid, tile);
+  const TilePos t = q8_tile_of(p.grid, tile, C::TileM);
   const TileSeg seg = q8_seg_of(p.grid, t.s);
   const int s0 = split * p.sk.per, s1 = min(p.steps, s0 + p.sk.per);
 
-  const int lrow4 = lane >> 2, chunk = lane & 3;
-  const int ra = 32 * wave + lrow4;
-  const __amdgpu_buffer_rsrc_t rA = q8_buffer(p.a + (long long)t.m0 * p.arow, (long long)min(kQ8TileM, p.m - t.m0) * p.arow);
-  const int offA0 = (int)(ra * p.arow) + ((chunk ^ q8_swizzle(ra)) << 4);
-  const int offA1 = (int)((ra + 16) * p.arow) + ((chunk ^ q8_swizzle(ra + 16)) << 4);
+  // blocks of 8 rows: lane l row l / 8, its 16 bytes chunk (l % 8) ^ (l / 8) of the stage's 128; the second step of a
+  // pair past s1 reads zeros (an offset past the buffers)
+  const int row8 = lane >> 3, chunk = (lane & 7) ^ row8;
+  const __amdgpu_buffer_rsrc_t rA = q8_buffer(p.a + (long long)t.m0 * p.arow, (long long)min(C::TileM, p.m - t.m0) * p.arow);
   const int rb0 = 16 * wave;
   const int colB = t.swiglu ? t.n0 + (rb0 & 63) : t.n0 + rb0;
   const unsigned char *wmat = (const unsigned char *)((t.swiglu && rb0 >= 64) ? seg.w3 : seg.w);
   const long long brow = seg.ldw * 4;
   const __amdgpu_buffer_rsrc_t rB = q8_buffer(wmat + (long long)colB * brow, (long long)min(16, seg.n - colB) * brow);
-  const int offB = (int)(lrow4 * brow) + ((chunk ^ q8_swizzle(lrow4)) << 4);
+  int offA[4], offB[2]; // per block (MI of A): the bounds check sees the lane's offset alone
+#pragma unroll
+  for (int i = 0; i < MI; i++)
+    offA[i] = (int)((8 * (MI * wave + i) + row8) * p.arow) + (chunk << 4);
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+    offB[i] = (int)((8 * i + row8) * brow) + (chunk << 4);
   const __amdgpu_buffer_rsrc_t none = q8_buffer(p.a, 0);
 
+  // steps `step` (even) and step + 1 into stage ST
   auto issue = [&](int step, auto ST) {
     constexpr int st = decltype(ST)::value;
-    const bool live = step < s1;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rA : none, (void *)(q8_smem + ((2 * wave) * kX3Stages + st) * 1024),
-                                             16, offA0, step * 64, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rA : none,
-                                             (void *)(q8_smem + ((2 * wave + 1) * kX3Stages + st) * 1024), 16, offA1,
-                                             step * 64, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rB : none,
-                                             (void *)(q8_smem + kX3BOff + (wave * kX3Stages + st) * 1024), 16, offB,
-                                             step * 64, 0, 0);
+    const bool live = step < s1, past = step + 1 >= s1 && chunk >= 4;
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rA : none,
+                                               (void *)(q8_smem + ((MI * wave + i) * C::Stages + st) * 1024), 16,
+                                               past ? 0x7FFFFFF0 : offA[i], step * 64, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rB : none,
+                                               (void *)(q8_smem + C::BOff + ((2 * wave + i) * C::Stages + st) * 1024), 16,
+                                               past ? 0x7FFFFFF0 : offB[i], step * 64, 0, 0);
   };
 
+  // lane (row r = l % 16, group q = l / 16) reads chunks q (first step) and 4 + q (second), held at chunk ^ (r % 8)
   const int lrow = lane & 15, lq = lane >> 4;
-  const int lane_part = lrow * 64 + ((lq ^ q8_swizzle(lrow)) << 4);
-  const unsigned char *abase = q8_smem + (4 * wm) * kX3Stages * 1024 + lane_part;
-  const unsigned char *bbase[4];
+  const int row_part = (lrow >> 3) * C::Stages * 1024 + (lrow & 7) * 128;
+  const int part[2] = {row_part + ((lq ^ (lrow & 7)) << 4), row_part + (((4 + lq) ^ (lrow & 7)) << 4)};
+  const unsigned char *abase = q8_smem + 2 * MI * wm * C::Stages * 1024, *bbase[4];
 #pragma unroll
   for (int j = 0; j < 4; j++)
-    bbase[j] = q8_smem + kX3BOff + (b_row(t.swiglu, wn, j) / 16) * kX3Stages * 1024 + lane_part;
+    bbase[j] = q8_smem + C::BOff + (b_row(t.swiglu, wn, j) / 8) * C::Stages * 1024;
 
-  v4f acc[4][4];
+  v4f acc[MI][4];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++)
       acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
   struct Operands {
-    v4f a[4], b[4];
+    v4f a[MI], b[4];
   };
-  auto operands = [&](auto ST, Operands &o) {
-    constexpr int st = decltype(ST)::value;
+  auto operands = [&](auto ST, auto H, Operands &o) {
+    constexpr int st = decltype(ST)::value, h = decltype(H)::value;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-      o.a[i] = *reinterpret_cast<const v4f *>(abase + (i * kX3Stages + st) * 1024);
+    for (int i = 0; i < MI; i++)
+      o.a[i] = *reinterpret_cast<const v4f *>(abase + part[h] + (2 * i * C::Stages + st) * 1024);
 #pragma unroll
     for (int j = 0; j < 4; j++)
-      o.b[j] = *reinterpret_cast<const v4f *>(bbase[j] + st * 1024);
+      o.b[j] = *reinterpret_cast<const v4f *>(bbase[j] + part[h] + st * 1024);
   };
   // the high halves of the three parts of x and y, packed: x in the low half of each dword
   struct Parts2 {
@@ -1180,14 +1216,14 @@ __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_f32x3(MmParams p) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, a), __builtin_bit_cast(v8bf_t, b), c, 0,
                                                     0, 0);
   };
-  // A pair's operands as BF16 parts: dwords 0 and 1 of each part from the first step's four values (split at the
-  // first step, while the previous pair's MFMAs drain), dwords 2 and 3 from the second's
+  // A pair's operands as BF16 parts: dwords 0 and 1 of each part from the first step's four values, 2 and 3 from the
+  // second's
   struct PairParts {
-    v4i_t ah[4], am[4], al[4], bh[4], bm[4], bl[4];
+    v4i_t ah[MI], am[MI], al[MI], bh[4], bm[4], bl[4];
   };
   auto split_half = [&](const Operands &o, PairParts &pp, int half) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < MI; i++) {
       const Parts2 lo = parts2(o.a[i][0], o.a[i][1]), hi = parts2(o.a[i][2], o.a[i][3]);
       pp.ah[i][2 * half] = lo.h, pp.ah[i][2 * half + 1] = hi.h;
       pp.am[i][2 * half] = lo.m, pp.am[i][2 * half + 1] = hi.m;
@@ -1204,7 +1240,7 @@ __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_f32x3(MmParams p) {
   // the MFMAs of a pair: the small products first
   auto mfmas3 = [&](const PairParts &pp) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < MI; i++) {
 #pragma unroll
       for (int j = 0; j < 4; j++)
         acc[i][j] = mfma(pp.al[i], pp.bh[j], acc[i][j]);
@@ -1226,42 +1262,36 @@ __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_f32x3(MmParams p) {
     }
   };
 
-  // As mm_gemm_lds: step + 1's loads have landed once only the later steps' may be outstanding, the barrier makes that
-  // true of every wave and frees the stage step - 1 used, which step + 5 now fills; the operands of step + 1 are read
-  // a step ahead. An even stage splits its step's half of the pair, an odd stage the other half and runs the MFMAs.
+  // The pair in stage ST, its first step's operands in `cur`: the second step's are read and both halves split; then
+  // every wave is done with the stage, the next pair has landed once only those after it may be outstanding, the pair
+  // Stages further fills the stage, and the next pair's first operands are read while the MFMAs run.
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, 1> second{};
   Operands cur, next;
   PairParts pp;
   auto advance = [&](int step, auto ST) {
-    constexpr int st = decltype(ST)::value, nst = (st + 1) % kX3Stages, fill = (st + kX3Stages - 1) % kX3Stages;
-    wait_vmcnt<(kX3Stages - 3) * kMmLoadsPerStep>();
-    __builtin_amdgcn_s_barrier();
-    issue(step + kX3Stages - 1, std::integral_constant<int, fill>{});
-    operands(std::integral_constant<int, nst>{}, next);
+    constexpr int nst = (decltype(ST)::value + 1) % C::Stages;
+    operands(ST, second, next);
     __builtin_amdgcn_sched_barrier(0);
-    split_half(cur, pp, st % 2);
-    if constexpr (st % 2 == 1) {
-      mfmas3(pp);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    cur = next;
+    split_half(cur, pp, 0);
+    split_half(next, pp, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt_lgkm0<(C::Stages - 2) * C::Loads>();
+    __builtin_amdgcn_s_barrier();
+    issue(step + 2 * C::Stages, ST);
+    operands(std::integral_constant<int, nst>{}, first, cur);
+    __builtin_amdgcn_sched_barrier(0);
+    mfmas3(pp);
+    __builtin_amdgcn_sched_barrier(0);
   };
 
-  issue(s0, std::integral_constant<int, 0>{});
-  issue(s0 + 1, std::integral_constant<int, 1>{});
-  issue(s0 + 2, std::integral_constant<int, 2>{});
-  issue(s0 + 3, std::integral_constant<int, 3>{});
-  issue(s0 + 4, std::integral_constant<int, 4>{});
-  wait_vmcnt<(kX3Stages - 2) * kMmLoadsPerStep>();
+  issue_first_pairs<0, C::Stages>(issue, s0);
+  wait_vmcnt<(C::Stages - 1) * C::Loads>();
   __builtin_amdgcn_s_barrier();
-  operands(std::integral_constant<int, 0>{}, cur);
-  for (int step = s0; step < s1; step += kX3Stages) {
-    advance(step, std::integral_constant<int, 0>{});
-    advance(step + 1, std::integral_constant<int, 1>{});
-    advance(step + 2, std::integral_constant<int, 2>{});
-    advance(step + 3, std::integral_constant<int, 3>{});
-    advance(step + 4, std::integral_constant<int, 4>{});
-    advance(step + 5, std::integral_constant<int, 5>{});
-  }
+  operands(std::integral_constant<int, 0>{}, first, cur);
+  for (int step = s0; step < s1; step += 2 * C::Stages) // as in bf16_gemm_lds
+    if (!pair_round<0, C::Stages, (MI <= 2)>(advance, step, s1))
+      break;
   __builtin_amdgcn_s_waitcnt(0);
   if (p.sk.splits > kCombineSplits) {
     store_partial(p.sk, tile, split, acc);
@@ -2022,11 +2052,11 @@ bool launch_ok(const char *what) {
   return raise("launching %s failed: %s", what, hipGetErrorString(e));
 }
 
-template <int J, int THREADS> bool launch_split_reduce(const Q8Grid &grid, const SplitK &sk, int m, int tile_m,
-                                                       int tile_n, hipStream_t stream) {
+template <int J, int THREADS, int MI = 4>
+bool launch_split_reduce(const Q8Grid &grid, const SplitK &sk, int m, int tile_m, int tile_n, hipStream_t stream) {
   SplitOut o{grid, sk.partial, sk.splits, m, tile_m, tile_n};
-  const long long threads = 4LL * (J / 2) * THREADS * grid.total;
-  hipLaunchKernelGGL((split_reduce<J, THREADS>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, o);
+  const long long threads = (long long)MI * (J / 2) * THREADS * grid.total;
+  hipLaunchKernelGGL((split_reduce<J, THREADS, MI>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, o);
   return launch_ok("split_reduce");
 }
 
@@ -2402,42 +2432,66 @@ bool f32_on_bf16_parts() {
   return !form || strcmp(form, "fp32") != 0;
 }
 
-// The partial tiles of a split FP32 / BF16 launch added up, where its blocks did not do that themselves.
-bool mm_reduce(const MmParams &p, hipStream_t stream) {
-  return p.sk.splits <= kCombineSplits ||
-         launch_split_reduce<4, kQ8Threads>(p.grid, p.sk, p.m, kQ8TileM, kQ8TileN, stream);
+// 16-row MFMA tiles per wave (a quarter of a block's rows) of the FP32 / BF16 kernels: the fewest that hold the batch in
+// as many row tiles as 256-row blocks take.
+int mm_row_tiles(int m) {
+  const int blocks = (m - 1) / kQ8TileM + 1;
+  return ((m - 1) / blocks + 64) / 64;
 }
 
-bool x3_launch(MmParams p, hipStream_t stream) {
-  static const hipError_t status =
-      hipFuncSetAttribute((const void *)mm_gemm_f32x3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kX3Lds);
-  if (!check_hip(status, "allowing the FP32 GEMM on BF16 parts its LDS"))
-    return false;
-  p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, p.steps, &p.sk.per);
+// The grid of 64 MI x 128 tiles and its splits. A split's steps are whole stages (two steps), or whole rounds of them
+// where the kernel runs whole rounds (512 x 3072 x 3072 BF16: four of 24 steps 31.4 us, five of 20, which run 24 each,
+// 32.9).
+MmParams mm_grid(MmParams p, const GemmF32Job &job, int mi, int unit) {
+  p.grid = make_q8_grid(job.seg, job.nseg, job.m, 64 * mi);
+  p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, p.steps, &p.sk.per, unit);
   if (p.sk.splits == 1)
     p.sk.per = p.steps;
   p.sk.partial = (v4f *)device().split_partial;
   p.sk.count = device().split_count;
-  hipLaunchKernelGGL(mm_gemm_f32x3, dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), kX3Lds, stream, p);
-  return launch_ok("mm_gemm_f32x3") && mm_reduce(p, stream);
+  return p;
 }
 
-// The FP32-product kernel, or the BF16 one, whose K loop runs whole rounds of its stages, two steps each: so do its
-// splits (512 x 3072 x 3072: four of 24 steps 31.4 us, five of 20, which run 24 each, 32.9).
-template <bool F32> bool mm_launch(MmParams p, hipStream_t stream) {
-  const auto kernel = F32 ? mm_gemm_lds : bf16_gemm_lds;
-  constexpr size_t lds = F32 ? kMmLds : kBfLds;
+// The partial tiles of a split launch added up, where its blocks did not do that themselves.
+template <int MI> bool mm_reduce(const MmParams &p, hipStream_t stream) {
+  return p.sk.splits <= kCombineSplits ||
+         launch_split_reduce<4, kQ8Threads, MI>(p.grid, p.sk, p.m, 64 * MI, kQ8TileN, stream);
+}
+
+// The BF16 kernel (panel rows, packed weights), or the FP32 one on BF16 parts, with 64 MI-row tiles.
+template <int MI, bool F32> bool mm_tile_launch(const MmParams &job_params, const GemmF32Job &job, hipStream_t stream) {
+  using C = MmTile<MI>;
   static const hipError_t status =
-      hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      F32 ? hipFuncSetAttribute((const void *)mm_gemm_f32x3<C>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::Lds)
+          : hipFuncSetAttribute((const void *)bf16_gemm_lds<C>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::Lds);
   if (!check_hip(status, "allowing the FP32 / BF16 GEMM its LDS"))
     return false;
-  p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, p.steps, &p.sk.per, F32 ? 1 : 2 * kBfStages);
-  if (p.sk.splits == 1)
-    p.sk.per = p.steps;
-  p.sk.partial = (v4f *)device().split_partial;
-  p.sk.count = device().split_count;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), lds, stream, p);
-  return launch_ok(F32 ? "mm_gemm_lds" : "bf16_gemm_lds") && mm_reduce(p, stream);
+  const MmParams p = mm_grid(job_params, job, MI, MI <= 2 ? 2 : 2 * C::Stages);
+  const dim3 grid((unsigned)(p.grid.total * p.sk.splits));
+  if (F32)
+    hipLaunchKernelGGL((mm_gemm_f32x3<C>), grid, dim3(kQ8Threads), C::Lds, stream, p);
+  else
+    hipLaunchKernelGGL((bf16_gemm_lds<C>), grid, dim3(kQ8Threads), C::Lds, stream, p);
+  return launch_ok(F32 ? "mm_gemm_f32x3" : "bf16_gemm_lds") && mm_reduce<MI>(p, stream);
+}
+
+template <bool F32> bool mm_tiles_launch(const MmParams &p, const GemmF32Job &job, hipStream_t stream) {
+  switch (mm_row_tiles(job.m)) {
+  case 1: return mm_tile_launch<1, F32>(p, job, stream);
+  case 2: return mm_tile_launch<2, F32>(p, job, stream);
+  case 3: return mm_tile_launch<3, F32>(p, job, stream);
+  default: return mm_tile_launch<4, F32>(p, job, stream);
+  }
+}
+
+bool f32_products_launch(const MmParams &job_params, const GemmF32Job &job, hipStream_t stream) {
+  static const hipError_t status =
+      hipFuncSetAttribute((const void *)mm_gemm_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMmLds);
+  if (!check_hip(status, "allowing the FP32 GEMM its LDS"))
+    return false;
+  const MmParams p = mm_grid(job_params, job, 4, 1);
+  hipLaunchKernelGGL(mm_gemm_lds, dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), kMmLds, stream, p);
+  return launch_ok("mm_gemm_lds") && mm_reduce<4>(p, stream);
 }
 
 // The wide BF16 kernel (256 x 256 tiles); its partial tiles are twice the size, so half as many fit the workspace.
@@ -2531,13 +2585,13 @@ bool launch_f32_gemm(const GemmF32Job &job, hipStream_t stream) {
     p.a = (const unsigned char *)job.panel;
     p.arow = (long long)kp * 2;
     p.steps = kp / 32;
-    return bf16_wide(p.grid.total) ? wide_launch(p, job, stream) : mm_launch<false>(p, stream);
+    return bf16_wide(p.grid.total) ? wide_launch(p, job, stream) : mm_tiles_launch<false>(p, job, stream);
   }
   if (f32_fast_path(job)) {
     p.a = (const unsigned char *)job.a;
     p.arow = (long long)job.lda * 4;
     p.steps = job.k / 16;
-    return f32_on_bf16_parts() ? x3_launch(p, stream) : mm_launch<true>(p, stream);
+    return f32_on_bf16_parts() ? mm_tiles_launch<true>(p, job, stream) : f32_products_launch(p, job, stream);
   }
   F32Params f{};
   f.grid = make_grid(job.seg, job.nseg, job.m);

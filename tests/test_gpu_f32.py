@@ -395,3 +395,51 @@ def test_bf16_gemm_odd_steps_and_neighbours(m, n, k):
         L.llhip_set_gemm_splits(0)
         L.llhip_set_bf16_tile(0)
         L.aligned_buffer_free(panel)
+
+
+@pytest.mark.parametrize("m", [1, 63, 64, 65, 128, 129, 192, 193, 256, 257, 333, 400, 513])
+@pytest.mark.parametrize("mode", ["bf16", "f32"])
+def test_gemm_row_tiles(mode, m):
+    """The FP32 and BF16 kernels take 64, 128, 192 or 256 rows a tile by the batch: every kind and split form (partial
+    tiles added in the last block and by the second kernel) at batches on both sides of each, a column tile
+    and its remainder, K steps that leave a stage half empty, and a second row of A infinite beside the finite ones. Budgets as in
+    test_gemm_split_k_all_kinds: 2e-5 (FP32) and 2e-6 (BF16 operands) of sum|a w|."""
+    L = hu.lib()
+    L.llhip_set_bf16_tile(1)
+    n, k = 72, 16 * 23 if mode == "f32" else 32 * 23
+    rng = orc.Rng(orc.SEED + 131 * m + len(mode))
+    a = rng.uniform(m * k, 2.0).reshape(m, k)
+    a[1::7] = np.inf
+    fine = np.isfinite(a[:, 0])
+    w, w3 = rng.uniform(n * k).reshape(n, k), rng.uniform(n * k).reshape(n, k)
+    base = rng.uniform(m * n, 4.0).reshape(m, n)
+    da, panel = hu.dev(a), lh.AlignedBuffer()
+    if mode == "bf16":
+        pw, pw3 = (np.zeros(L.bf16_vnni_elements(n, k), np.uint16) for _ in range(2))
+        L.pack_bf16_vnni(lh.ptr(pw), lh.ptr(w), n, k, k)
+        L.pack_bf16_vnni(lh.ptr(pw3), lh.ptr(w3), n, k, k)
+        dw, dw3 = hu.dev(pw), hu.dev(pw3)
+        ab, wb, w3b = bf16_round(a[fine].copy()), bf16_round(w), bf16_round(w3)
+        (r, mag), (r3, mag3), rel = ref_f32(ab, wb), ref_f32(ab, w3b), 2e-6
+        L.aligned_buffer_alloc(panel, L.k_gemm_bf16_panel_bytes(m, k), 1)
+    else:
+        dw, dw3 = hu.dev(w), hu.dev(w3)
+        (r, mag), (r3, mag3), rel = ref_f32(a[fine], w), ref_f32(a[fine], w3), 2e-5
+    try:
+        for kind in (lh.GEMM_STORE, lh.GEMM_ADD, lh.GEMM_SWIGLU):
+            for splits in (1, 2, 5):
+                L.llhip_set_gemm_splits(splits)
+                c = hu.dev(base)
+                if mode == "bf16":
+                    seg = lh.GemmBf16Segment(lh.ptr(c), n, lh.ptr(dw), lh.ptr(dw3), n, kind)
+                    L.k_gemm_bf16(lh.ptr(da), k, m, k, seg, 1, panel)
+                else:
+                    seg = lh.GemmSegment(lh.ptr(c), n, lh.ptr(dw), lh.ptr(dw3), k, n, kind)
+                    L.k_gemm_f32(lh.ptr(da), k, m, k, seg, 1)
+                check_kind(hu.host(c)[fine], base[fine], r, mag, r3, mag3, kind, rel=rel,
+                           what=f"{mode} {m} rows kind {kind} splits {splits}")
+    finally:
+        L.llhip_set_gemm_splits(0)
+        L.llhip_set_bf16_tile(0)
+        if mode == "bf16":
+            L.aligned_buffer_free(panel)
