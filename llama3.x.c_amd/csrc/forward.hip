@@ -790,7 +790,7 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash(Att
   bool bad = false;
   const bool split = p.splits > 0; // block (tile, g, s) takes share s of the tile's chunks and stores a partial
   for (int pass = 0; pass < 2; pass++) {
-    const int tile = split ? (int)blockIdx.x : pass == 0 ? ntiles - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    const int tile = pass == 0 ? ntiles - 1 - (int)blockIdx.x : (int)blockIdx.x; // the longest walks start first
     if (pass == 1 && (split || tile >= ntiles - 1 - (int)blockIdx.x))
       break; // the middle tile of an odd count is taken once
     const int r0 = tile * tile_rows, row = r0 + j;
@@ -1084,7 +1084,7 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash3(At
   bool bad = false, qbad = false;
   const bool split = p.splits > 0;
   for (int pass = 0; pass < 2; pass++) {
-    const int tile = split ? (int)blockIdx.x : pass == 0 ? ntiles - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    const int tile = pass == 0 ? ntiles - 1 - (int)blockIdx.x : (int)blockIdx.x; // the longest walks start first
     if (pass == 1 && (split || tile >= ntiles - 1 - (int)blockIdx.x))
       break;
     const int r0 = tile * tile_rows, row = r0 + j;
@@ -1501,7 +1501,9 @@ __global__ __launch_bounds__(kThreads) void attn_merge(AttnParams p) {
 // maxima (a share that held no chunk stores -FLT_MAX and zero sums), weights exp(m_s - M) in share order, and the
 // output sum_s w_s o_s / sum_s w_s l_s. The same combination as attn_merge with the sums in share order; with at most
 // 16 shares a thread needs no reduction across the block, so the grid is as small as the output.
-__global__ __launch_bounds__(kThreads) void attn_merge_shares(AttnParams p) {
+// S: the shares' count rounded up to 2, 4, 8 or 16, every load of a thread in flight at once (a share past the count
+// repeats the last one and is not taken).
+template <int S> __global__ __launch_bounds__(kThreads) void attn_merge_shares(AttnParams p) {
   const int q4 = p.head_dim / 4;
   const long long idx = (long long)blockIdx.x * kThreads + threadIdx.x;
   if (idx >= (long long)p.rows * p.n_heads * q4)
@@ -1510,18 +1512,28 @@ __global__ __launch_bounds__(kThreads) void attn_merge_shares(AttnParams p) {
   const long long rh = idx / q4; // row * n_heads + head
   const float *part = p.partial + (size_t)rh * p.splits * p.slot; // the slots of row * n_heads + head
   const int hd = p.head_dim;
+  float ms[S], ls[S];
+  float4 v[S];
+#pragma unroll
+  for (int s = 0; s < S; s++) {
+    const float *share = part + (size_t)min(s, p.splits - 1) * p.slot;
+    ms[s] = share[hd];
+    ls[s] = share[hd + 1];
+    v[s] = *reinterpret_cast<const float4 *>(share + 4 * d4);
+  }
   float m = -FLT_MAX;
-  for (int s = 0; s < p.splits; s++)
-    m = fmaxf(m, part[(size_t)s * p.slot + hd]);
+#pragma unroll
+  for (int s = 0; s < S; s++)
+    m = fmaxf(m, ms[s]);
   float4 o = float4{0.0f, 0.0f, 0.0f, 0.0f};
   float l = 0.0f;
-  for (int s = 0; s < p.splits; s++) {
-    const float *share = part + (size_t)s * p.slot;
-    const float w = expf(share[hd] - m);
-    l = fmaf(w, share[hd + 1], l);
-    const float4 v = *reinterpret_cast<const float4 *>(share + 4 * d4);
-    o = float4{fmaf(w, v.x, o.x), fmaf(w, v.y, o.y), fmaf(w, v.z, o.z), fmaf(w, v.w, o.w)};
-  }
+#pragma unroll
+  for (int s = 0; s < S; s++)
+    if (s < p.splits) {
+      const float w = expf(ms[s] - m);
+      l = fmaf(w, ls[s], l);
+      o = float4{fmaf(w, v[s].x, o.x), fmaf(w, v[s].y, o.y), fmaf(w, v[s].z, o.z), fmaf(w, v[s].w, o.w)};
+    }
   *reinterpret_cast<float4 *>(p.out + rh * hd + 4 * d4) = float4{o.x / l, o.y / l, o.z / l, o.w / l};
 }
 
@@ -1680,14 +1692,18 @@ bool attention_flash_bf3() {
   return !form || strcmp(form, "fp32") != 0;
 }
 
-// Blocks per tile of the batched kernel (0: one block per pair of tiles, no partials). A block walks its tiles' 64-position
-// chunks at about the same time per chunk whatever the grid, so a grid of few blocks with long walks (a short batch
-// late in a sequence: a prompt prefilled in batches) leaves most CUs idle for the whole walk. Split S gives each tile S
-// blocks over shares of its chunks and adds attn_merge_shares. The choice is the S in {1, 2, 4, 8, 16} of least
-// estimated time, with one 64-position walk taking the kernel's measured time (below): unsplit, the longest pair's
-// chunks times the rounds of the CUs its grid takes; split, the longest share's chunks times the rounds, plus the
-// merge; a split must save a tenth. Its partials stay within job.partial_room. LLAMA_HIP_FLASH_SPLITS = n forces n
-// (1: never split), for tuning and tests.
+// Blocks per tile of the batched kernel (0: one block per pair of tiles, no partials). A block walks its tiles' chunks at
+// about the same time per chunk whatever the grid, so a grid of few blocks with long walks (a prompt of some hundred
+// rows, or a short batch late in a sequence) leaves most CUs idle for the whole walk. Split S gives each tile S blocks
+// over shares of its chunks and adds attn_merge_shares. The choice is the S of least estimated time, `unit` positions
+// taking the kernel's measured time: unsplit, the longest pair's walk times the rounds of the CUs its grid takes; split,
+// the longest share, or where the blocks are more than the CUs the smaller of whole rounds of it and an even load plus
+// half of it (the shares of a causal batch differ, and the longest start first), plus the partials' cost. Fitted to
+// forced splits of twelve shapes, within a tenth of each (us, unsplit / chosen / best of 2 .. 16): 600 rows of 32 + 8
+// heads of 64 43 / 32 / 32 (left unsplit by an estimate of whole rounds alone), 300 rows 27 / 17 / 17, 512 rows of 24 + 8
+// heads of 128 66 / 35 / 35, 700 rows from position 300 133 / 68 / 68 (before 77), 256 rows of 32 + 8 from 1792 349 / 60 /
+// 60, 40 rows from 2000 362 / 25 / 25; 1024 rows 105 / 105 / 112. A split must save a twentieth. Its partials stay within
+// job.partial_room. LLAMA_HIP_FLASH_SPLITS = n forces n (1: never split), for tuning and tests.
 int flash_splits(const AttentionJob &job, int chunks) {
   const int kv_mul = job.n_heads / job.n_kv_heads;
   const int tile_rows = 128 / kv_mul, tiles = (job.rows + tile_rows - 1) / tile_rows;
@@ -1695,24 +1711,27 @@ int flash_splits(const AttentionJob &job, int chunks) {
   const char *env = getenv("LLAMA_HIP_FLASH_SPLITS");
   int splits = env && *env ? atoi(env) : 0;
   if (splits <= 0) {
-    auto walk = [&](int t) { return (job.pos0 + min((t + 1) * tile_rows, job.rows) - 1) / kChunk + 1; };
-    auto rounds = [&](long long blocks) { return (double)((blocks + cus - 1) / cus); };
-    // the BF16-part kernel walks a 64-position span in about 5.7 us at head_dim 128 (3.5 at 64), and its merge grows
-    // with the shares (each share's partials read and rescaled): fitted to forced splits of 128 to 512 rows at 8B, 3B
-    // and 1B heads; the FP32-product kernel's figures are the first ones measured
+    // the BF16-part kernel walks 32 positions in about 2.85 us at head_dim 128 (1.75 at 64); the FP32-product kernel's
+    // figures are for 64
     const bool bf3 = attention_flash_bf3();
-    const double chunk_us = bf3 ? (job.head_dim == 128 ? 5.7 : 3.5) : (job.head_dim == 128 ? 10.0 : 6.0);
-    auto merge = [&](int s) {
-      const double per_row = job.rows * job.n_heads / 32.0;
-      return bf3 ? 2.0 + 0.011 * per_row * s * job.head_dim / 128.0 : 2.0 + 0.012 * per_row;
+    const int unit = bf3 ? 32 : kChunk;
+    const double unit_us = (job.head_dim == 128 ? 1.0 : 0.61) * (bf3 ? 2.85 : 10.0);
+    auto walk = [&](int t) {
+      const long long end = (long long)(t + 1) * tile_rows;
+      return (int)((job.pos0 + (end < job.rows ? end : job.rows) - 1) / unit + 1);
     };
-    const int pairs = (tiles + 1) / 2;
-    const double unsplit = chunk_us * (walk(tiles - 1) + (tiles > 1 ? walk(0) : 0)) *
-                           rounds((long long)pairs * job.n_kv_heads);
-    double best = 0.9 * unsplit;
+    auto rounds = [&](long long blocks) { return (double)((blocks + cus - 1) / cus); };
+    const int first = walk(0), last = walk(tiles - 1);
+    const double even = 0.5 * (first + last) * tiles * job.n_kv_heads / cus; // every walk over the CUs
+    const double per_share = 0.011 * (job.rows * (double)job.n_heads / 32.0) * job.head_dim / 128.0;
+    const double unsplit = 5.0 + unit_us * (last + (tiles > 1 ? first : 0)) *
+                                     rounds((long long)((tiles + 1) / 2) * job.n_kv_heads);
+    double best = 0.95 * unsplit;
     splits = 1;
-    for (int s = 2; s <= 16; s *= 2) {
-      const double t = chunk_us * ((chunks + s - 1) / s) * rounds((long long)tiles * job.n_kv_heads * s) + merge(s);
+    for (int s : {2, 3, 4, 6, 8, 12, 16}) {
+      const double share = (last + s - 1) / s;
+      const double work = fmax(share, fmin(share * rounds((long long)tiles * job.n_kv_heads * s), even + 0.5 * share));
+      const double t = 5.0 + (job.qout ? 3.0 : 0.0) + unit_us * work + per_share * s; // 3: the rows' own quantization
       if (t < best)
         best = t, splits = s;
     }
@@ -1798,8 +1817,15 @@ bool launch_attention(const AttentionJob &job, float *partial, hipStream_t strea
       return false;
     if (p.splits) {
       const long long threads = (long long)job.rows * job.n_heads * (job.head_dim / 4);
-      hipLaunchKernelGGL(attn_merge_shares, dim3((unsigned)((threads + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                         stream, p);
+      const dim3 blocks((unsigned)((threads + kThreads - 1) / kThreads));
+      if (p.splits <= 2)
+        hipLaunchKernelGGL(attn_merge_shares<2>, blocks, dim3(kThreads), 0, stream, p);
+      else if (p.splits <= 4)
+        hipLaunchKernelGGL(attn_merge_shares<4>, blocks, dim3(kThreads), 0, stream, p);
+      else if (p.splits <= 8)
+        hipLaunchKernelGGL(attn_merge_shares<8>, blocks, dim3(kThreads), 0, stream, p);
+      else
+        hipLaunchKernelGGL(attn_merge_shares<16>, blocks, dim3(kThreads), 0, stream, p);
       if (!launch_ok("attn_merge_shares"))
         return false;
     }
