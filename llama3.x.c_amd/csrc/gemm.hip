@@ -4,6 +4,7 @@
 // ADD and SWIGLU (a column tile then holds columns of W1 and the same columns of W3, so the gate is applied in
 // registers). The kernels, each described where it is defined:
 //   q8_gemm_lds     int8, 256 x 128 tiles (or 128 x 128), A/B/scales streamed into LDS five stages deep;
+//   q8_gemm_rows    int8 with gs = 64, 64 to 256 rows a tile, two groups a stage;
 //   mm_gemm_lds     FP32, 256 x 128 tiles, the same pipeline;
 //   mm_gemm_f32x3   FP32 on the BF16 matrix cores, the default FP32 kernel;
 //   bf16_gemm_lds   BF16, 256 x 128 tiles, two K steps a stage;
@@ -136,13 +137,14 @@ __device__ __forceinline__ void store_tile(const TileSeg &seg, const TilePos &t,
 // reduction), the two meet in LDS (`xchg`, free once every wave has left the K loop), and each quantizes its values
 // with the group's scale by the k_quantize rule, as store_tile_wide does (bitwise the FP32 output then
 // k_quantize_rows); a non-finite value sets flags[0]. Every wave of the block calls it (two barriers).
-__device__ __forceinline__ void store_tile_quantized(const TileSeg &seg, const TilePos &t, const v4f (&acc)[4][4],
+template <int MI>
+__device__ __forceinline__ void store_tile_quantized(const TileSeg &seg, const TilePos &t, const v4f (&acc)[MI][4],
                                                      int wm, int wn, int lane, int m, float *xchg, int *flags) {
   const int lc = lane & 15, lr = (lane >> 4) * 4;
   // two passes over the sums (the SwiGLU values formed twice) so that only the sums stay live across the barriers
   __syncthreads(); // every wave is past its K loop: the LDS is free
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       float pk = 0.0f;
@@ -151,17 +153,17 @@ __device__ __forceinline__ void store_tile_quantized(const TileSeg &seg, const T
         pk = fmaxf(pk, fabsf(silu_gate(acc[i][j][e], acc[i][j + 2][e]))); // a NaN: caught by quantize_fast
       pk = group_reduce_max(pk, 16);
       if (lc == 0)
-        xchg[(wm * 64 + 16 * i + lr + e) * 2 + wn] = pk;
+        xchg[(wm * 16 * MI + 16 * i + lr + e) * 2 + wn] = pk;
     }
   __syncthreads();
   const int c0 = t.n0; // the tile's group (seg.n % 64 == 0)
   const int groups = seg.ldc / 64; // row strides of cq and cs: the whole width (a tail segment has its share)
   bool bad = false;
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int r = wm * 64 + 16 * i + lr + e, row = t.m0 + r;
+      const int r = wm * 16 * MI + 16 * i + lr + e, row = t.m0 + r;
       const float scale = fmaxf(xchg[r * 2], xchg[r * 2 + 1]) / 127.0f;
       bool ok;
       const float inv = group_reciprocal(scale, ok);
@@ -759,6 +761,200 @@ __global__ __launch_bounds__(C::Threads, 2) void q8_gemm_lds(Q8Params p) {
     return;
   }
   if constexpr (QUANT)
+    store_tile_quantized(seg, t, acc, wm, wn, lane, p.m, reinterpret_cast<float *>(q8_smem), p.flags);
+  else
+    store_tile(seg, t, acc, wm, wn, lane, p.m);
+}
+
+// ---- W8A8 Q8_0, gs = 64: two groups a stage, 64 to 256 rows a tile ---------------------------------------------------
+//
+// q8_gemm_lds's tile and arithmetic (the same expression in the same group order: unsplit, bit for bit its results) with
+// the row tiles and 128-byte stages of bf16_gemm_lds: a stage holds two groups, whole cache lines of each row, and a
+// block 256, 192, 128 or 64 rows by the batch, with more stages where the rows are few. Below 256 rows a tile the rows
+// past the batch cost most of the time (the rescale, then the MFMAs, take it in sequence: a SIMD does not overlap its
+// matrix and vector work); at 256 whole lines help while K is long. Measured, q8_gemm_lds / this (us): 40 x 2 * 14336 x
+// 4096 SwiGLU 65 / 44, 40 x 4096 x 14336 43 / 29, 100 x 2048 x 8192 26 / 21, 128 x 3072 x 3072 26 / 20, 333 x 2 * 8192 x
+// 3072 59 / 52, 2048 x 4096 x 14336 284 / 277.
+template <int MI_, int STAGES_> struct Q8RowsCfg {
+  static constexpr int MI = MI_, Stages = STAGES_, TileM = 64 * MI;
+  static constexpr int Loads = MI + 4;                  // per wave and stage: MI blocks of A, two of B, two of scales
+  static constexpr int BOff = 8 * MI * Stages * 1024;    // A: 8 MI blocks of 8 rows a stage, then 16 of B
+  static constexpr int SOff = BOff + 16 * Stages * 1024; // then the scales of each group: xs, ws, spare
+  static constexpr int SGroup = (TileM + kQ8TileN + 64) * 4, SStride = 2 * SGroup;
+  static constexpr size_t Lds = (size_t)SOff + (size_t)Stages * SStride;
+  static_assert(Lds <= 160 * 1024, "one int8 block fits a CU's LDS");
+};
+template <int MI> using Q8Rows = Q8RowsCfg<MI, MI == 1 ? 6 : MI == 2 ? 4 : 3>;
+
+template <class C, bool SPLIT, bool QUANT> __global__ __launch_bounds__(kQ8Threads, 2) void q8_gemm_rows(Q8Params p) {
+  constexpr int MI = C::MI;
+  extern __shared__ __align__(16) unsigned char q8_smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int logical = xcd_logical(blockIdx.x, p.grid.total * (SPLIT ? p.sk.splits : 1));
+  const int tile = SPLIT ? __builtin_amdgcn_readfirstlane(logical / p.sk.splits) : logical;
+  const int split = SPLIT ? __builtin_amdgcn_readfirstlane(logical % p.sk.splits) : 0;
+  const TilePos t = q8_tile_of(p.grid, tile, C::TileM);
+  const TileSeg seg = q8_seg_of(p.grid, t.s);
+  const int groups = p.k / 64;
+  const int s0 = SPLIT ? split * p.sk.per : 0, s1 = SPLIT ? min(groups, s0 + p.sk.per) : groups;
+  const long long k = p.k;
+
+  // Blocks of 8 rows: lane l takes row l / 8, its 16 bytes chunk (l % 8) ^ (l / 8) of the pair's 128. The second group
+  // of a pair past s1 reads zeros (an offset past the buffers: its bytes are the next row's, or the next split's).
+  const int row8 = lane >> 3, chunk = (lane & 7) ^ row8;
+  const __amdgpu_buffer_rsrc_t rA = q8_buffer(p.xq + (long long)t.m0 * k, (long long)min(C::TileM, p.m - t.m0) * k);
+  int offA[4], offB[2]; // per block (MI of A): the bounds check sees the lane's offset alone
+#pragma unroll
+  for (int i = 0; i < MI; i++)
+    offA[i] = (int)((8 * (MI * wave + i) + row8) * k) + (chunk << 4);
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+    offB[i] = (int)((8 * i + row8) * k) + (chunk << 4);
+  const int rb0 = 16 * wave; // B-tile rows of the wave's two blocks, all of one matrix
+  const int colB = t.swiglu ? t.n0 + (rb0 & 63) : t.n0 + rb0;
+  const int8_t *wmat = (const int8_t *)((t.swiglu && rb0 >= 64) ? seg.w3 : seg.w);
+  const __amdgpu_buffer_rsrc_t rB = q8_buffer(wmat + (long long)colB * k, (long long)min(16, seg.n - colB) * k);
+  // Scale loads, 64 a group: waves 0 .. MI - 1 the xs rows, the next two the ws rows, any others nothing (to the spare).
+  __amdgpu_buffer_rsrc_t rS;
+  int scale_dst;
+  if (wave < MI) {
+    const int r0 = t.m0 + 64 * wave;
+    rS = q8_buffer(p.xs + (long long)r0 * groups, (long long)min(64, p.m - r0) * groups * 4);
+    scale_dst = 64 * wave * 4;
+  } else if (wave < MI + 2) {
+    const int h = wave - MI;
+    const float *src = t.swiglu ? (h ? seg.w3s : seg.ws) : seg.ws;
+    const int c0 = t.swiglu ? t.n0 : t.n0 + 64 * h;
+    rS = q8_buffer(src + (long long)c0 * groups, (long long)min(64, seg.n - c0) * groups * 4);
+    scale_dst = (C::TileM + 64 * h) * 4;
+  } else {
+    rS = q8_buffer(p.xs, 0);
+    scale_dst = (C::TileM + kQ8TileN) * 4;
+  }
+  const int offS = lane * groups * 4;
+  const __amdgpu_buffer_rsrc_t none = q8_buffer(p.xq, 0);
+
+  // groups step and step + 1 into stage st
+  auto issue = [&](int step, int st) {
+    const bool live = step < s1, both = step + 1 < s1, past = !both && chunk >= 4;
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rA : none,
+                                               (void *)(q8_smem + ((MI * wave + i) * C::Stages + st) * 1024), 16,
+                                               past ? 0x7FFFFFF0 : offA[i], step * 64, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rB : none,
+                                               (void *)(q8_smem + C::BOff + ((2 * wave + i) * C::Stages + st) * 1024), 16,
+                                               past ? 0x7FFFFFF0 : offB[i], step * 64, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rS : none, (void *)(q8_smem + C::SOff + st * C::SStride + scale_dst), 4,
+                                             offS, step * 4, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        both ? rS : none, (void *)(q8_smem + C::SOff + st * C::SStride + C::SGroup + scale_dst), 4, offS, step * 4 + 4, 0,
+        0);
+  };
+
+  // Operand reads: lane (row r = l % 16, group q = l / 16) takes chunk 4 H + q of its row, held at (4 H + q) ^ (r % 8).
+  const int lrow = lane & 15, lq = lane >> 4, lr4 = lq * 4;
+  const int row_part = (lrow >> 3) * C::Stages * 1024 + (lrow & 7) * 128;
+  const int part[2] = {row_part + ((lq ^ (lrow & 7)) << 4), row_part + (((4 + lq) ^ (lrow & 7)) << 4)};
+  const unsigned char *abase = q8_smem + 2 * MI * wm * C::Stages * 1024, *bbase[4];
+  const unsigned char *xsbase = q8_smem + C::SOff + (wm * 16 * MI + lr4) * 4, *wsbase[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    bbase[j] = q8_smem + C::BOff + (b_row(t.swiglu, wn, j) / 8) * C::Stages * 1024;
+    wsbase[j] = q8_smem + C::SOff + (C::TileM + b_row(t.swiglu, wn, j) + lrow) * 4;
+  }
+  struct Operands {
+    v4i a[MI], b[4];
+  };
+  struct Scales {
+    v4f xs[MI];
+    float ws[4];
+  };
+  auto operands = [&](int st, int h, Operands &o) {
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+      o.a[i] = *reinterpret_cast<const v4i *>(abase + (part[h] + st * 1024) + 2 * i * C::Stages * 1024);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      o.b[j] = *reinterpret_cast<const v4i *>(bbase[j] + (part[h] + st * 1024));
+  };
+  auto scales = [&](int st, int h, Scales &s) {
+    const int at = st * C::SStride + h * C::SGroup;
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+      s.xs[i] = *reinterpret_cast<const v4f *>(xsbase + at + i * 64);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      s.ws[j] = *reinterpret_cast<const float *>(wsbase[j] + at);
+  };
+
+  v4f acc[MI][4];
+  v4i dot[MI][4];
+#pragma unroll
+  for (int i = 0; i < MI; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  // Tile by tile: the pending group's int32 results converted, the next group's MFMA over them, the rescale added.
+  auto rescale_and_mfma = [&](const Operands &o, const Scales &s) {
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        float f[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          f[e] = (float)dot[i][j][e];
+        dot[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a[i], o.b[j], v4i{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          acc[i][j][e] = fmaf(f[e] * s.ws[j], s.xs[i][e], acc[i][j][e]);
+      }
+  };
+
+#pragma unroll
+  for (int st = 0; st < C::Stages; st++)
+    issue(s0 + 2 * st, st);
+  wait_vmcnt<(C::Stages - 1) * C::Loads>();
+  __builtin_amdgcn_s_barrier();
+  {
+    Operands o;
+    operands(0, 0, o);
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        dot[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a[i], o.b[j], v4i{0, 0, 0, 0}, 0, 0, 0);
+  }
+  // The pair in stage st, its first group's MFMAs done: the second's while the first is rescaled; then every wave has
+  // read the stage, the next pair has landed once only those after it may be outstanding, the pair Stages further fills
+  // the stage, and the next pair's first MFMAs run while the second group is rescaled. After the last pair they run on
+  // stale operands whose products are never used. The stage is a variable, an add per base address and pair: a loop
+  // unrolled by the stages either leaves inside a round, which keeps the sums twice and spilled 100 registers a lane, or
+  // runs whole rounds of six groups.
+  for (int step = s0, st = 0; step < s1; step += 2) {
+    const int nst = st + 1 == C::Stages ? 0 : st + 1;
+    Operands o;
+    Scales sc;
+    operands(st, 1, o);
+    scales(st, 0, sc);
+    rescale_and_mfma(o, sc);
+    scales(st, 1, sc);
+    wait_vmcnt_lgkm0<(C::Stages - 2) * C::Loads>();
+    __builtin_amdgcn_s_barrier();
+    issue(step + 2 * C::Stages, st);
+    operands(nst, 0, o);
+    rescale_and_mfma(o, sc);
+    st = nst;
+  }
+  __builtin_amdgcn_s_waitcnt(0); // loads issued for pairs past the end still target this block's LDS
+  if constexpr (SPLIT)
+    store_partial(p.sk, tile, split, acc);
+  else if constexpr (QUANT)
     store_tile_quantized(seg, t, acc, wm, wn, lane, p.m, reinterpret_cast<float *>(q8_smem), p.flags);
   else
     store_tile(seg, t, acc, wm, wn, lane, p.m);
@@ -2092,6 +2288,13 @@ Q8Grid make_q8_grid(const GemmSegmentDev *segs, int nseg, int m, int tile_m = kQ
   return g;
 }
 
+// 16-row MFMA tiles per wave (a quarter of a block's rows) of the kernels with 64 to 256 rows
+// a tile: the fewest that hold the batch in as many row tiles as 256-row blocks take.
+int row_tiles(int m) {
+  const int blocks = (m - 1) / kQ8TileM + 1;
+  return ((m - 1) / blocks + 64) / 64;
+}
+
 std::atomic<int> forced_splits{0};
 
 // Blocks per tile: one when the tiles fill the CUs (one 256 x 128 block per CU fits in LDS), else enough to reach
@@ -2121,6 +2324,44 @@ template <class C, bool PROBE, bool GS64, bool SPLIT, bool QUANT = false> bool q
   return check_hip(status, "allowing the Q8 GEMM its LDS");
 }
 
+// gs = 64 with 64 MI-row tiles.
+template <int MI, bool QUANT> bool q8_rows_launch(Q8Params p, const SegList &segs, hipStream_t stream) {
+  using C = Q8Rows<MI>;
+  static const hipError_t whole = hipFuncSetAttribute((const void *)q8_gemm_rows<C, false, QUANT>,
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::Lds);
+  static const hipError_t parts = hipFuncSetAttribute((const void *)q8_gemm_rows<C, true, false>,
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::Lds);
+  if (!check_hip(whole, "allowing the Q8 GEMM its LDS") || !check_hip(parts, "allowing the Q8 GEMM its LDS"))
+    return false;
+  p.grid = make_q8_grid(segs.seg, segs.nseg, p.m, C::TileM);
+  if (p.grid.total <= 0)
+    return true;
+  const int steps = p.k / 64;
+  p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, steps, &p.sk.per);
+  p.sk.partial = (v4f *)device().split_partial;
+  p.sk.count = device().split_count;
+  if (p.sk.splits == 1) {
+    p.sk.per = steps;
+    hipLaunchKernelGGL((q8_gemm_rows<C, false, QUANT>), dim3((unsigned)p.grid.total), dim3(kQ8Threads), C::Lds, stream, p);
+    return launch_ok("q8_gemm_rows");
+  }
+  if (QUANT) // the quantized epilogue has no split form
+    return raise("q8_gemm_rows: a quantized SwiGLU output cannot be split");
+  hipLaunchKernelGGL((q8_gemm_rows<C, true, false>), dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), C::Lds,
+                     stream, p);
+  return launch_ok("q8_gemm_rows") &&
+         launch_split_reduce<4, kQ8Threads, MI>(p.grid, p.sk, p.m, C::TileM, kQ8TileN, stream);
+}
+
+template <bool QUANT> bool q8_rows(const Q8Params &p, const SegList &segs, hipStream_t stream) {
+  switch (row_tiles(p.m)) {
+  case 1: return q8_rows_launch<1, QUANT>(p, segs, stream);
+  case 2: return q8_rows_launch<2, QUANT>(p, segs, stream);
+  case 3: return q8_rows_launch<3, QUANT>(p, segs, stream);
+  default: return q8_rows_launch<4, QUANT>(p, segs, stream);
+  }
+}
+
 template <class C, bool PROBE, bool GS64, bool QUANT = false>
 bool q8_launch(Q8Params p, const SegList &segs, hipStream_t stream) {
   p.grid = make_q8_grid(segs.seg, segs.nseg, p.m, C::TileM);
@@ -2128,6 +2369,11 @@ bool q8_launch(Q8Params p, const SegList &segs, hipStream_t stream) {
     return true;
   const int steps = p.k / 64;
   p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, steps, &p.sk.per, p.gs / 64);
+  // gs = 64: fewer than 256 rows a tile, or whole 256-row tiles. 256-row tiles split over short K ranges stay here (256 x
+  // 6144 x 4096 30.6 us, 32.2 in q8_gemm_rows; 600 x 2048 x 8192 42.9 / 45.0; 1000 x 3072 x 8192 87.6 / 91.0).
+  if constexpr (GS64 && !PROBE && C::WM == 4)
+    if (p.sk.splits == 1 || row_tiles(p.m) < 4)
+      return q8_rows<QUANT>(p, segs, stream);
   if (p.sk.splits == 1)
     p.sk.per = steps;
   p.sk.partial = (v4f *)device().split_partial;
@@ -2432,13 +2678,6 @@ bool f32_on_bf16_parts() {
   return !form || strcmp(form, "fp32") != 0;
 }
 
-// 16-row MFMA tiles per wave (a quarter of a block's rows) of the FP32 / BF16 kernels: the fewest that hold the batch in
-// as many row tiles as 256-row blocks take.
-int mm_row_tiles(int m) {
-  const int blocks = (m - 1) / kQ8TileM + 1;
-  return ((m - 1) / blocks + 64) / 64;
-}
-
 // The grid of 64 MI x 128 tiles and its splits. A split's steps are whole stages (two steps), or whole rounds of them
 // where the kernel runs whole rounds (512 x 3072 x 3072 BF16: four of 24 steps 31.4 us, five of 20, which run 24 each,
 // 32.9).
@@ -2476,7 +2715,7 @@ template <int MI, bool F32> bool mm_tile_launch(const MmParams &job_params, cons
 }
 
 template <bool F32> bool mm_tiles_launch(const MmParams &p, const GemmF32Job &job, hipStream_t stream) {
-  switch (mm_row_tiles(job.m)) {
+  switch (row_tiles(job.m)) {
   case 1: return mm_tile_launch<1, F32>(p, job, stream);
   case 2: return mm_tile_launch<2, F32>(p, job, stream);
   case 3: return mm_tile_launch<3, F32>(p, job, stream);

@@ -919,3 +919,48 @@ def test_fused_quantization_with_output_over_its_input():
     L.k_matmul_q8_add(lh.ptr(xd), lh.k8(qd, sd, xd), lh.w8(dwq, dws), n, d, gs)
     hu.assert_within_budget(hu.host(xd), x + ref, mag + np.abs(x), what="residual over the quantized input")
     assert np.array_equal(hu.host(qd), xq)
+
+
+@pytest.mark.parametrize("m", [33, 63, 64, 65, 128, 129, 192, 193, 256, 257, 333, 513])
+@pytest.mark.parametrize("k", [64, 192, 1216])
+def test_gemm_q8_row_tiles(m, k):
+    """gs = 64 tiles of 64 to 256 rows by the batch (q8_gemm_rows), two groups a stage: batches on both sides of each tile
+    height, odd group counts (a stage's second group empty), K ranges of a split that begin and end inside a cache line;
+    every kind within the budget, and with one block per tile bit for bit the 256 x 256 kernel's vector-unit form, which
+    adds the same terms in the same order."""
+    L = hu.lib()
+    gs, n = 64, 88
+    xq, xs, wq, ws, w3q, w3s, rng = gemm_case(m, n, k, gs, 5100 + m + k)
+    base = rng.uniform(m * n, 3.0).reshape(m, n)
+    ref, mag = hu.dequant_reference(xq, xs, wq, ws, gs)
+    r3, mag3 = hu.dequant_reference(xq, xs, w3q, w3s, gs)
+    dx = [hu.dev(a) for a in (xq, xs, wq, ws, w3q, w3s)]
+
+    def run(kind, tile, splits):
+        L.llhip_set_q8_tile(tile)
+        L.llhip_set_gemm_splits(splits)
+        c = hu.dev(base)
+        seg = lh.GemmQ8Segment(lh.ptr(c), n, lh.w8(dx[2], dx[3]), lh.w8(dx[4], dx[5]), None, None, n, kind)
+        L.k_gemm_q8(lh.ptr(dx[0]), lh.ptr(dx[1]), m, k, gs, seg, 1)
+        got = hu.host(c)
+        assert lh.last_error() == "", lh.last_error()
+        return got
+
+    try:
+        L.llhip_set_q8_scales(1)
+        for kind in (lh.GEMM_STORE, lh.GEMM_ADD, lh.GEMM_SWIGLU):
+            for splits in (1, 3, 0):
+                got, what = run(kind, 1, splits), f"{m}x{n}x{k} kind {kind} splits {splits}"
+                if kind == lh.GEMM_ADD:
+                    hu.assert_within_budget(got, base + ref, mag + np.abs(base), what=what)
+                elif kind == lh.GEMM_SWIGLU:
+                    tol = 2e-5 * (mag * (np.abs(r3) + 1) + mag3 * (np.abs(ref) + 1)) + 1e-6  # tests/q8.c:130
+                    assert np.all(np.abs(got - ref / (1 + np.exp(-ref)) * r3) <= tol), what
+                else:
+                    hu.assert_within_budget(got, ref, mag, what=what)
+                if splits == 1:
+                    assert np.array_equal(hu.bits(got), hu.bits(run(kind, 2, 1))), what + " vs 256 x 256"
+    finally:
+        L.llhip_set_q8_tile(0)
+        L.llhip_set_gemm_splits(0)
+        L.llhip_set_q8_scales(0)
