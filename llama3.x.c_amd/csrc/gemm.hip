@@ -2353,8 +2353,39 @@ template <int MI, bool QUANT> bool q8_rows_launch(Q8Params p, const SegList &seg
          launch_split_reduce<4, kQ8Threads, MI>(p.grid, p.sk, p.m, C::TileM, kQ8TileN, stream);
 }
 
-template <bool QUANT> bool q8_rows(const Q8Params &p, const SegList &segs, hipStream_t stream) {
-  switch (row_tiles(p.m)) {
+// Tile height (in 64-row units) of a gs = 64 GEMM whose 256-row grid leaves CUs idle: row_tiles, or another where the
+// estimate below is a tenth better. A lower tile has more tiles, so fewer blocks a tile, and its partial tiles are
+// smaller; but each of its blocks takes more than its share of a 256-row block's time. Fitted to forced heights (us a
+// group; a split launch 6 us and its partials at 2.5 TB/s, else 3) and measured, chosen / row_tiles' (us): 256 x 4096 x
+// 4096 25.3 (128 rows) / 29.4, 600 x 3072 x 2048 21.0 (64 rows, unsplit) / 30.0, 600 x 2048 x 2048 23.6 / 26.2, 600 x 2048
+// x 8192 41.5 / 42.9.
+int q8_tile_height(const Q8Params &p, const SegList &segs) {
+  const int base = row_tiles(p.m);
+  if (forced_splits.load() > 0)
+    return base;
+  const int cus = device().cu_count > 0 ? device().cu_count : 256, steps = p.k / 64;
+  auto estimate = [&](int mi) {
+    static const double group_us[4] = {0.52, 0.72, 0.97, 1.25};
+    const int tiles = make_q8_grid(segs.seg, segs.nseg, p.m, 64 * mi).total;
+    int per = steps;
+    const int splits = tiles > kSplitSlots ? 1 : choose_splits(tiles, steps, &per);
+    const int blocks = tiles * splits;
+    return (double)((blocks + cus - 1) / cus) * (splits > 1 ? per : steps) * group_us[mi - 1] +
+           (splits > 1 ? 6.0 + blocks * mi * 32.768e-3 / 2.5 : 3.0);
+  };
+  double best = 0.9 * estimate(base);
+  int height = base;
+  for (int mi = 1; mi <= 4; mi++)
+    if (mi != base) {
+      const double t = estimate(mi);
+      if (t < best)
+        best = t, height = mi;
+    }
+  return height;
+}
+
+template <bool QUANT> bool q8_rows(int height, const Q8Params &p, const SegList &segs, hipStream_t stream) {
+  switch (height) {
   case 1: return q8_rows_launch<1, QUANT>(p, segs, stream);
   case 2: return q8_rows_launch<2, QUANT>(p, segs, stream);
   case 3: return q8_rows_launch<3, QUANT>(p, segs, stream);
@@ -2371,9 +2402,11 @@ bool q8_launch(Q8Params p, const SegList &segs, hipStream_t stream) {
   p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, steps, &p.sk.per, p.gs / 64);
   // gs = 64: fewer than 256 rows a tile, or whole 256-row tiles. 256-row tiles split over short K ranges stay here (256 x
   // 6144 x 4096 30.6 us, 32.2 in q8_gemm_rows; 600 x 2048 x 8192 42.9 / 45.0; 1000 x 3072 x 8192 87.6 / 91.0).
-  if constexpr (GS64 && !PROBE && C::WM == 4)
-    if (p.sk.splits == 1 || row_tiles(p.m) < 4)
-      return q8_rows<QUANT>(p, segs, stream);
+  if constexpr (GS64 && !PROBE && C::WM == 4) {
+    const int height = QUANT ? row_tiles(p.m) : q8_tile_height(p, segs);
+    if (p.sk.splits == 1 || height < 4)
+      return q8_rows<QUANT>(height, p, segs, stream);
+  }
   if (p.sk.splits == 1)
     p.sk.per = steps;
   p.sk.partial = (v4f *)device().split_partial;

@@ -964,3 +964,34 @@ def test_gemm_q8_row_tiles(m, k):
         L.llhip_set_q8_tile(0)
         L.llhip_set_gemm_splits(0)
         L.llhip_set_q8_scales(0)
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 512, 512), (320, 640, 1024), (600, 384, 2048), (700, 96, 640), (100, 256, 2048)])
+def test_gemm_q8_chosen_tile_height(m, n, k):
+    """Short grids of a gs = 64 GEMM choose their tile height and split together: every kind within the budget, the same
+    bits on a repeated call, and nothing written past the columns."""
+    L = hu.lib()
+    gs, ldc = 64, n + 5
+    xq, xs, wq, ws, w3q, w3s, rng = gemm_case(m, n, k, gs, 5300 + m + n)
+    base = rng.uniform(m * ldc, 3.0).reshape(m, ldc)
+    ref, mag = hu.dequant_reference(xq, xs, wq, ws, gs)
+    r3, mag3 = hu.dequant_reference(xq, xs, w3q, w3s, gs)
+    dx = [hu.dev(a) for a in (xq, xs, wq, ws, w3q, w3s)]
+    for kind in (lh.GEMM_STORE, lh.GEMM_ADD, lh.GEMM_SWIGLU):
+        got = []
+        for _ in range(2):
+            c = hu.dev(base)
+            seg = lh.GemmQ8Segment(lh.ptr(c), ldc, lh.w8(dx[2], dx[3]), lh.w8(dx[4], dx[5]), None, None, n, kind)
+            L.k_gemm_q8(lh.ptr(dx[0]), lh.ptr(dx[1]), m, k, gs, seg, 1)
+            got.append(hu.host(c))
+            assert lh.last_error() == "", lh.last_error()
+        assert np.array_equal(hu.bits(got[0]), hu.bits(got[1]))
+        assert np.array_equal(hu.bits(got[0][:, n:]), hu.bits(base[:, n:])), "row padding was written"
+        out, what = got[0][:, :n], f"{m}x{n}x{k} kind {kind}"
+        if kind == lh.GEMM_ADD:
+            hu.assert_within_budget(out, base[:, :n] + ref, mag + np.abs(base[:, :n]), what=what)
+        elif kind == lh.GEMM_SWIGLU:
+            tol = 2e-5 * (mag * (np.abs(r3) + 1) + mag3 * (np.abs(ref) + 1)) + 1e-6  # tests/q8.c:130
+            assert np.all(np.abs(out - ref / (1 + np.exp(-ref)) * r3) <= tol), what
+        else:
+            hu.assert_within_budget(out, ref, mag, what=what)
