@@ -2066,12 +2066,18 @@ template <bool SPLIT> __global__ __launch_bounds__(kQ8Threads, 2) void q8_gemm_w
       }
       if (j < 7)
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0); // the next round's DS reads
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // the scale-product MFMA
+      // the other set's 32 converts and FMAs spread over the round, eight behind the scale products' 32 cycles: the first
+      // int8 MFMA right behind them kept the wave waiting (QKV of 2048 rows 118 -> 115 us, 4096 x 4096 x 14336 479 -> 470)
+      if (j > 0 || carry)
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // the scale-product MFMA
+      if (j > 0 || carry)
+        __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // one int8 MFMA
         if (j > 0 || carry)
-          __builtin_amdgcn_sched_group_barrier(0x002, 8, 0); // one tile's convert and FMA
+          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0); // converts and FMAs
       }
       if (sst >= 0 && j == 3) {
         __builtin_amdgcn_sched_group_barrier(0x002, 8, 0); // splitting the scale
