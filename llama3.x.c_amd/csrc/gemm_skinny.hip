@@ -137,7 +137,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void q8_gemm_skinny(SkParams p) {
   // Weights two K steps at a time: load X takes rows 0-7 and Y rows 8-15, each row's 128 bytes whole (lane l: row
   // l % 8, 16-byte chunk l / 16 + 4 ((l % 16) / 8), so lanes 0-7 of each 16-lane row hold the first step's chunk and
   // lanes 8-15 the second's). A pair may reach past the wave's range or the row's end: the activations of such a step
-  // read zero, so whatever weight bytes it holds add nothing.
+  // read zero, so whatever weight bytes it holds (those past the row's end: zeros) add nothing.
   const int chunk = (lane >> 4) + 4 * ((lane >> 3) & 1);
   const int offX = (int)((lane & 7) * k) + 16 * chunk, offY = offX + (int)(8 * k);
 
@@ -145,13 +145,16 @@ __global__ __launch_bounds__(64 * WAVES, 2) void q8_gemm_skinny(SkParams p) {
   auto issue = [&](int st, int d) { // steps st and st + 1
     const bool live = st < s1;
     const int k0 = st * 64;
+    // the second step of a pair past the row's end is not read (behind the last row lies the end of the weights)
+    const bool past = st + 1 >= p.steps && chunk >= 4;
+    const int ox = past ? 0x7FFFFFF0 : offX, oy = past ? 0x7FFFFFF0 : offY;
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-      x[d][j] = __builtin_amdgcn_raw_buffer_load_b128(live ? rB[j] : none, offX, k0, kStream);
-      y[d][j] = __builtin_amdgcn_raw_buffer_load_b128(live ? rB[j] : none, offY, k0, kStream);
+      x[d][j] = __builtin_amdgcn_raw_buffer_load_b128(live ? rB[j] : none, ox, k0, kStream);
+      y[d][j] = __builtin_amdgcn_raw_buffer_load_b128(live ? rB[j] : none, oy, k0, kStream);
       if constexpr (SW) {
-        x3[d][j] = __builtin_amdgcn_raw_buffer_load_b128(live ? rB3[j] : none, offX, k0, kStream);
-        y3[d][j] = __builtin_amdgcn_raw_buffer_load_b128(live ? rB3[j] : none, offY, k0, kStream);
+        x3[d][j] = __builtin_amdgcn_raw_buffer_load_b128(live ? rB3[j] : none, ox, k0, kStream);
+        y3[d][j] = __builtin_amdgcn_raw_buffer_load_b128(live ? rB3[j] : none, oy, k0, kStream);
       }
     }
 #pragma unroll
