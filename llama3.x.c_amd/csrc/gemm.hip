@@ -137,14 +137,13 @@ __device__ __forceinline__ void store_tile(const TileSeg &seg, const TilePos &t,
 // reduction), the two meet in LDS (`xchg`, free once every wave has left the K loop), and each quantizes its values
 // with the group's scale by the k_quantize rule, as store_tile_wide does (bitwise the FP32 output then
 // k_quantize_rows); a non-finite value sets flags[0]. Every wave of the block calls it (two barriers).
-template <int MI>
-__device__ __forceinline__ void store_tile_quantized(const TileSeg &seg, const TilePos &t, const v4f (&acc)[MI][4],
+__device__ __forceinline__ void store_tile_quantized(const TileSeg &seg, const TilePos &t, const v4f (&acc)[4][4],
                                                      int wm, int wn, int lane, int m, float *xchg, int *flags) {
   const int lc = lane & 15, lr = (lane >> 4) * 4;
   // two passes over the sums (the SwiGLU values formed twice) so that only the sums stay live across the barriers
   __syncthreads(); // every wave is past its K loop: the LDS is free
 #pragma unroll
-  for (int i = 0; i < MI; i++)
+  for (int i = 0; i < 4; i++)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       float pk = 0.0f;
@@ -153,17 +152,17 @@ __device__ __forceinline__ void store_tile_quantized(const TileSeg &seg, const T
         pk = fmaxf(pk, fabsf(silu_gate(acc[i][j][e], acc[i][j + 2][e]))); // a NaN: caught by quantize_fast
       pk = group_reduce_max(pk, 16);
       if (lc == 0)
-        xchg[(wm * 16 * MI + 16 * i + lr + e) * 2 + wn] = pk;
+        xchg[(wm * 64 + 16 * i + lr + e) * 2 + wn] = pk;
     }
   __syncthreads();
   const int c0 = t.n0; // the tile's group (seg.n % 64 == 0)
   const int groups = seg.ldc / 64; // row strides of cq and cs: the whole width (a tail segment has its share)
   bool bad = false;
 #pragma unroll
-  for (int i = 0; i < MI; i++)
+  for (int i = 0; i < 4; i++)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int r = wm * 16 * MI + 16 * i + lr + e, row = t.m0 + r;
+      const int r = wm * 64 + 16 * i + lr + e, row = t.m0 + r;
       const float scale = fmaxf(xchg[r * 2], xchg[r * 2 + 1]) / 127.0f;
       bool ok;
       const float inv = group_reciprocal(scale, ok);
@@ -766,15 +765,19 @@ __global__ __launch_bounds__(C::Threads, 2) void q8_gemm_lds(Q8Params p) {
     store_tile(seg, t, acc, wm, wn, lane, p.m);
 }
 
-// ---- W8A8 Q8_0, gs = 64: two groups a stage, 64 to 256 rows a tile ---------------------------------------------------
+// ---- W8A8 Q8_0, gs = 64: two groups a stage, 64 to 192 rows a tile ---------------------------------------------------
 //
 // q8_gemm_lds's tile and arithmetic (the same expression in the same group order: unsplit, bit for bit its results) with
-// the row tiles and 128-byte stages of bf16_gemm_lds: a stage holds two groups, whole cache lines of each row, and a
-// block 256, 192, 128 or 64 rows by the batch, with more stages where the rows are few. Below 256 rows a tile the rows
-// past the batch cost most of the time (the rescale, then the MFMAs, take it in sequence: a SIMD does not overlap its
-// matrix and vector work); at 256 whole lines help while K is long. Measured, q8_gemm_lds / this (us): 40 x 2 * 14336 x
-// 4096 SwiGLU 65 / 44, 40 x 4096 x 14336 43 / 29, 100 x 2048 x 8192 26 / 21, 128 x 3072 x 3072 26 / 20, 333 x 2 * 8192 x
-// 3072 59 / 52, 2048 x 4096 x 14336 284 / 277.
+// the row tiles and 128-byte stages of bf16_gemm_lds: a stage holds two groups, 128 bytes of each row, and a block 192,
+// 128 or 64 rows by the batch, with more stages where the rows are few. A row's 128 bytes are one whole cache line where
+// the block's K range begins at an even group; a split's range may begin at an odd one, and its lines then hold half of
+// two stages each. In 256-row tiles the rows past the batch cost their share of the MFMAs and the rescale all the same.
+// Measured, q8_gemm_lds / this (us): 40 x 2 * 14336 x 4096 SwiGLU 65 / 44, 40 x 4096 x 14336 43 / 29, 100 x 2048 x 8192
+// 26 / 21, 128 x 3072 x 3072 26 / 20, 333 x 2 * 8192 x 3072 59 / 52.
+// 256-row tiles stay with q8_gemm_lds. A form of this kernel for them halved the loads that reach L2 (2048 x 3072 x 8192:
+// 18.8 to 10.0 million) but waits at its barrier for the operands it reads right behind it (waves' waiting cycles 24 to
+// 32 million): 2048 x 3072 x 8192 125 / 134 us, 1024 x 6144 x 4096 68 / 73, 256 x 2 * 14336 x 4096 72 / 74, 3 to 8% slower
+// wherever the last round of tiles leaves CUs idle, and within 2% where every CU has one (2048 x 4096 x 14336 243 / 239).
 template <int MI_, int STAGES_> struct Q8RowsCfg {
   static constexpr int MI = MI_, Stages = STAGES_, TileM = 64 * MI;
   static constexpr int Loads = MI + 4;                  // per wave and stage: MI blocks of A, two of B, two of scales
@@ -782,11 +785,11 @@ template <int MI_, int STAGES_> struct Q8RowsCfg {
   static constexpr int SOff = BOff + 16 * Stages * 1024; // then the scales of each group: xs, ws, spare
   static constexpr int SGroup = (TileM + kQ8TileN + 64) * 4, SStride = 2 * SGroup;
   static constexpr size_t Lds = (size_t)SOff + (size_t)Stages * SStride;
-  static_assert(Lds <= 160 * 1024, "one int8 block fits a CU's LDS");
+  static_assert(MI < 4 && Lds <= 160 * 1024, "one int8 block fits a CU's LDS");
 };
 template <int MI> using Q8Rows = Q8RowsCfg<MI, MI == 1 ? 6 : MI == 2 ? 4 : 3>;
 
-template <class C, bool SPLIT, bool QUANT> __global__ __launch_bounds__(kQ8Threads, 2) void q8_gemm_rows(Q8Params p) {
+template <class C, bool SPLIT> __global__ __launch_bounds__(kQ8Threads, 2) void q8_gemm_rows(Q8Params p) {
   constexpr int MI = C::MI;
   extern __shared__ __align__(16) unsigned char q8_smem[];
   const int lane = threadIdx.x & 63;
@@ -954,12 +957,9 @@ template <class C, bool SPLIT, bool QUANT> __global__ __launch_bounds__(kQ8Threa
   __builtin_amdgcn_s_waitcnt(0); // loads issued for pairs past the end still target this block's LDS
   if constexpr (SPLIT)
     store_partial(p.sk, tile, split, acc);
-  else if constexpr (QUANT)
-    store_tile_quantized(seg, t, acc, wm, wn, lane, p.m, reinterpret_cast<float *>(q8_smem), p.flags);
   else
     store_tile(seg, t, acc, wm, wn, lane, p.m);
 }
-
 
 // Round to nearest even on the 16 dropped bits, NaN quieted with its sign and top payload bits, denormals kept,
 // overflow to infinity: the conversion of the reference's bf16_from_f32 (src/gemm.c:335-342), as an integer formula.
@@ -2331,11 +2331,11 @@ template <class C, bool PROBE, bool GS64, bool SPLIT, bool QUANT = false> bool q
 }
 
 // gs = 64 with 64 MI-row tiles.
-template <int MI, bool QUANT> bool q8_rows_launch(Q8Params p, const SegList &segs, hipStream_t stream) {
+template <int MI> bool q8_rows_launch(Q8Params p, const SegList &segs, hipStream_t stream) {
   using C = Q8Rows<MI>;
-  static const hipError_t whole = hipFuncSetAttribute((const void *)q8_gemm_rows<C, false, QUANT>,
+  static const hipError_t whole = hipFuncSetAttribute((const void *)q8_gemm_rows<C, false>,
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::Lds);
-  static const hipError_t parts = hipFuncSetAttribute((const void *)q8_gemm_rows<C, true, false>,
+  static const hipError_t parts = hipFuncSetAttribute((const void *)q8_gemm_rows<C, true>,
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::Lds);
   if (!check_hip(whole, "allowing the Q8 GEMM its LDS") || !check_hip(parts, "allowing the Q8 GEMM its LDS"))
     return false;
@@ -2348,23 +2348,20 @@ template <int MI, bool QUANT> bool q8_rows_launch(Q8Params p, const SegList &seg
   p.sk.count = device().split_count;
   if (p.sk.splits == 1) {
     p.sk.per = steps;
-    hipLaunchKernelGGL((q8_gemm_rows<C, false, QUANT>), dim3((unsigned)p.grid.total), dim3(kQ8Threads), C::Lds, stream, p);
+    hipLaunchKernelGGL((q8_gemm_rows<C, false>), dim3((unsigned)p.grid.total), dim3(kQ8Threads), C::Lds, stream, p);
     return launch_ok("q8_gemm_rows");
   }
-  if (QUANT) // the quantized epilogue has no split form
-    return raise("q8_gemm_rows: a quantized SwiGLU output cannot be split");
-  hipLaunchKernelGGL((q8_gemm_rows<C, true, false>), dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), C::Lds,
+  hipLaunchKernelGGL((q8_gemm_rows<C, true>), dim3((unsigned)(p.grid.total * p.sk.splits)), dim3(kQ8Threads), C::Lds,
                      stream, p);
   return launch_ok("q8_gemm_rows") &&
          launch_split_reduce<4, kQ8Threads, MI>(p.grid, p.sk, p.m, C::TileM, kQ8TileN, stream);
 }
 
-// Tile height (in 64-row units) of a gs = 64 GEMM whose 256-row grid leaves CUs idle: row_tiles, or another where the
-// estimate below is a tenth better. A lower tile has more tiles, so fewer blocks a tile, and its partial tiles are
-// smaller; but each of its blocks takes more than its share of a 256-row block's time. Fitted to forced heights (us a
-// group; a split launch 6 us and its partials at 2.5 TB/s, else 3) and measured, chosen / row_tiles' (us): 256 x 4096 x
-// 4096 25.3 (128 rows) / 29.4, 600 x 3072 x 2048 21.0 (64 rows, unsplit) / 30.0, 600 x 2048 x 2048 23.6 / 26.2, 600 x 2048
-// x 8192 41.5 / 42.9.
+// Tile height (in 64-row units) of a gs = 64 GEMM: row_tiles, or another where the estimate below is a tenth better. A
+// lower tile has more tiles, so fewer blocks a tile, and its partial tiles are smaller; but each of its blocks takes more
+// than its share of a 256-row block's time. Fitted to forced heights (us a group; a split launch 6 us and its partials at
+// 2.5 TB/s, else 3) and measured, chosen / row_tiles' (us): 256 x 4096 x 4096 25.3 (128 rows) / 29.4, 600 x 3072 x 2048
+// 21.0 (64 rows, unsplit) / 30.0, 600 x 2048 x 2048 23.6 / 26.2, 600 x 2048 x 8192 41.5 / 42.9.
 int q8_tile_height(const Q8Params &p, const SegList &segs) {
   const int base = row_tiles(p.m);
   if (forced_splits.load() > 0)
@@ -2390,12 +2387,11 @@ int q8_tile_height(const Q8Params &p, const SegList &segs) {
   return height;
 }
 
-template <bool QUANT> bool q8_rows(int height, const Q8Params &p, const SegList &segs, hipStream_t stream) {
+bool q8_rows(int height, const Q8Params &p, const SegList &segs, hipStream_t stream) {
   switch (height) {
-  case 1: return q8_rows_launch<1, QUANT>(p, segs, stream);
-  case 2: return q8_rows_launch<2, QUANT>(p, segs, stream);
-  case 3: return q8_rows_launch<3, QUANT>(p, segs, stream);
-  default: return q8_rows_launch<4, QUANT>(p, segs, stream);
+  case 1: return q8_rows_launch<1>(p, segs, stream);
+  case 2: return q8_rows_launch<2>(p, segs, stream);
+  default: return q8_rows_launch<3>(p, segs, stream);
   }
 }
 
@@ -2406,12 +2402,10 @@ bool q8_launch(Q8Params p, const SegList &segs, hipStream_t stream) {
     return true;
   const int steps = p.k / 64;
   p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, steps, &p.sk.per, p.gs / 64);
-  // gs = 64: fewer than 256 rows a tile, or whole 256-row tiles. 256-row tiles split over short K ranges stay here (256 x
-  // 6144 x 4096 30.6 us, 32.2 in q8_gemm_rows; 600 x 2048 x 8192 42.9 / 45.0; 1000 x 3072 x 8192 87.6 / 91.0).
-  if constexpr (GS64 && !PROBE && C::WM == 4) {
-    const int height = QUANT ? row_tiles(p.m) : q8_tile_height(p, segs);
-    if (p.sk.splits == 1 || height < 4)
-      return q8_rows<QUANT>(height, p, segs, stream);
+  if constexpr (GS64 && !PROBE && !QUANT && C::WM == 4) { // gs = 64: fewer than 256 rows a tile
+    const int height = q8_tile_height(p, segs);
+    if (height < 4)
+      return q8_rows(height, p, segs, stream);
   }
   if (p.sk.splits == 1)
     p.sk.per = steps;
