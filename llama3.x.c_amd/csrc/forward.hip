@@ -1703,7 +1703,8 @@ bool attention_flash_bf3() {
 // heads of 64 43 / 32 / 32 (left unsplit by an estimate of whole rounds alone), 300 rows 27 / 17 / 17, 512 rows of 24 + 8
 // heads of 128 66 / 35 / 35, 700 rows from position 300 133 / 68 / 68 (before 77), 256 rows of 32 + 8 from 1792 349 / 60 /
 // 60, 40 rows from 2000 362 / 25 / 25; 1024 rows 105 / 105 / 112. A split must save a twentieth. Its partials stay within
-// job.partial_room. LLAMA_HIP_FLASH_SPLITS = n forces n (1: never split), for tuning and tests.
+// job.partial_room. The choice never looks at job.qout: quantized rows are bitwise the FP32 rows quantized, so both calls walk the
+// same shares. LLAMA_HIP_FLASH_SPLITS = n forces n (1: never split), for tuning and tests.
 int flash_splits(const AttentionJob &job, int chunks) {
   const int kv_mul = job.n_heads / job.n_kv_heads;
   const int tile_rows = 128 / kv_mul, tiles = (job.rows + tile_rows - 1) / tile_rows;
@@ -1731,7 +1732,7 @@ int flash_splits(const AttentionJob &job, int chunks) {
     for (int s : {2, 3, 4, 6, 8, 12, 16}) {
       const double share = (last + s - 1) / s;
       const double work = fmax(share, fmin(share * rounds((long long)tiles * job.n_kv_heads * s), even + 0.5 * share));
-      const double t = 5.0 + (job.qout ? 3.0 : 0.0) + unit_us * work + per_share * s; // 3: the rows' own quantization
+      const double t = 5.0 + unit_us * work + per_share * s;
       if (t < best)
         best = t, splits = s;
     }

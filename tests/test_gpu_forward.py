@@ -337,7 +337,7 @@ def test_attention_flash_fp32_form(shape, monkeypatch):
 
 
 @pytest.mark.parametrize("nh,nkv,hd,seq,pos0,m,gs,layout,form", [
-    (32, 8, 128, 600, 0, 512, 64, "head", None),      # 8B heads: quantized in the flash kernel's epilogue
+    (32, 8, 128, 600, 0, 512, 64, "head", None),      # 8B heads, split: merged, then quantized
     (24, 8, 128, 300, 10, 100, 32, "rows", None),     # kv_mul 3 (idle vectors), groups of 32
     (32, 8, 64, 300, 0, 130, 64, "head", None),       # 64 dimensions, a group per head
     (16, 4, 128, 200, 3, 40, 128, "head", None),      # a group of a whole head
@@ -370,6 +370,18 @@ def test_attention_batch_quantize_fused(nh, nkv, hd, seq, pos0, m, gs, layout, f
         assert np.array_equal(hu.bits(hu.host(xs)), hu.bits(hu.host(xs2)))
     finally:
         assert L.kernels_kv_layout_select(b"head") == 1
+
+
+@pytest.mark.parametrize("splits", [0, 1, 3])
+@pytest.mark.parametrize("nh,nkv,hd,m,gs", [(32, 8, 128, 862, 64), (24, 8, 128, 1345, 32), (32, 8, 64, 900, 64),
+                                           (32, 8, 128, 1024, 128)])
+def test_attention_batch_quantize_same_shares(nh, nkv, hd, m, gs, splits, monkeypatch):
+    """The quantizing call walks the shares that the FP32 call walks (0: as chosen, at batches near the line between an
+    unsplit and a split grid; 1: unsplit, so the flash kernel quantizes in its epilogue; 3: merged, then quantized), so
+    the rows are bitwise the FP32 rows quantized."""
+    if splits:
+        monkeypatch.setenv("LLAMA_HIP_FLASH_SPLITS", str(splits))
+    test_attention_batch_quantize_fused(nh, nkv, hd, m + 3, 0, m, gs, "head", None, monkeypatch)
 
 
 @pytest.mark.parametrize("splits,shape", [(3, (16, 8, 128, 400, 130, 77, "head")), (16, (32, 8, 128, 600, 0, 512, "head")),
