@@ -307,6 +307,7 @@ struct AttnParams {
   size_t pos_stride, head_base;
   float divisor; // sqrtf(head_dim)
   int splits;    // batched flash form: blocks per tile, each over a share of its chunks (0: the tile whole)
+  bool by_length; // split: the blocks listed from the longest walk to the shortest
   // attn_flash3 unsplit: the output rows quantized in groups of qgs values (k_quantize) instead of stored in FP32
   int8_t *qout;
   float *qscale;
@@ -769,6 +770,23 @@ template <int HD> struct FlashDma {
 // s_waitcnt vmcnt(0): this wave's loads, LDS DMA included, are complete
 __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// The work of a batched block. Unsplit: blocks (rank, g) take the rank-th tile from the end, then the rank-th from the
+// start. Split: blocks (rank, g, share), or, where they outnumber the CUs (by_length), one dimension of them: tile by
+// tile from the end, a tile's shares over every KV head together, so the longest walks start first and consecutive
+// blocks, which go to the XCDs in turn, are equally long; the heads turn by one a tile, so an XCD has all of them at any
+// time. With the tiles as the fastest index, one XCD had all of the longest tiles where the tiles are a multiple of eight
+// (2048 rows of 4 heads of 128 in six shares 82 us, listed 48; 1024 rows of 32 + 8 heads in two 112 / 74). Where every
+// block starts at once nothing is gained (333 rows of 24 + 8 heads 22.6 us, listed 25.4; 256 rows of 32 + 8 21.4 / 23.4).
+struct FlashBlock {
+  int rank, g, share;
+};
+__device__ __forceinline__ FlashBlock flash_block(const AttnParams &p) {
+  if (!p.by_length)
+    return FlashBlock{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
+  const int walks = p.n_kv_heads * p.splits, rank = (int)blockIdx.x / walks, w = (int)blockIdx.x % walks;
+  return FlashBlock{rank, (w + rank) % p.n_kv_heads, w / p.n_kv_heads};
+}
+
 template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash(AttnParams p) {
   constexpr int kQ = HD / 4;       // dimensions per lane group in the score MFMAs
   constexpr int kDt = HD / 16;     // 16-dimension tiles of the value sums
@@ -779,7 +797,9 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash(Att
   __shared__ __align__(16) float K0[kChunk * kSt], K1[kChunk * kSt], V0[kChunk * kSt], V1[kChunk * kSt];
   const int kv_mul = p.n_heads / p.n_kv_heads, tile_rows = kQv / kv_mul;
   const int ntiles = (p.rows + tile_rows - 1) / tile_rows;
-  const int g = blockIdx.y;
+  const bool split = p.splits > 0;
+  const FlashBlock at = flash_block(p);
+  const int g = at.g;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int lq = lane >> 4, lc = lane & 15;
   const int qv = wave * 16 + lc, j = qv / kv_mul, h = qv % kv_mul;
@@ -788,10 +808,9 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash(Att
   // scores in base 2: s * log2(e) / divisor, so that exp(s / divisor - m) is the native exp2 of (s2 - m2)
   const float scale2 = 1.4426950408889634f / p.divisor;
   bool bad = false;
-  const bool split = p.splits > 0; // block (tile, g, s) takes share s of the tile's chunks and stores a partial
   for (int pass = 0; pass < 2; pass++) {
-    const int tile = pass == 0 ? ntiles - 1 - (int)blockIdx.x : (int)blockIdx.x; // the longest walks start first
-    if (pass == 1 && (split || tile >= ntiles - 1 - (int)blockIdx.x))
+    const int tile = pass == 0 ? ntiles - 1 - at.rank : at.rank; // the longest walks start first
+    if (pass == 1 && (split || tile >= ntiles - 1 - at.rank))
       break; // the middle tile of an odd count is taken once
     const int r0 = tile * tile_rows, row = r0 + j;
     // vectors past tile_rows * kv_mul (when kv_mul does not divide 128) would be the next tile's: idle, like rows past
@@ -944,7 +963,7 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash(Att
     // V((c + 1) % 2), last read for chunk c - 1, takes chunk c + 1.
     // this block's chunks: c0 .. c0 + chunks - 1 (all of the tile's unless split)
     const int all = last / kChunk + 1, share = split ? (all + p.splits - 1) / p.splits : all;
-    const int c0 = split ? min(all, (int)blockIdx.z * share) : 0, chunks = min(all, c0 + share) - c0;
+    const int c0 = split ? min(all, at.share * share) : 0, chunks = min(all, c0 + share) - c0;
     v4f sc[4];
     auto step = [&](int c, const float *kn, float *kdma, const float *vs, float *vdma) {
       const int t0 = (c0 + c) * kChunk;
@@ -986,7 +1005,7 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash(Att
       continue;
     if (split) { // the share's value sums, maximum (in natural units, as the merge takes it) and sum, unnormalized;
       // slots [row][head][share]: rows x n_heads x splits x slot floats in all, the room flash_splits checked
-      float *slot = p.partial + (((size_t)row * p.n_heads + (size_t)g * kv_mul + h) * p.splits + blockIdx.z) * p.slot;
+      float *slot = p.partial + (((size_t)row * p.n_heads + (size_t)g * kv_mul + h) * p.splits + at.share) * p.slot;
 #pragma unroll
       for (int e = 0; e < 4; e++)
 #pragma unroll
@@ -1046,7 +1065,9 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash3(At
   __shared__ __align__(16) uint16_t Vp[2][3 * kVPart];
   const int kv_mul = p.n_heads / p.n_kv_heads, tile_rows = kQv / kv_mul;
   const int ntiles = (p.rows + tile_rows - 1) / tile_rows;
-  const int g = blockIdx.y;
+  const bool split = p.splits > 0;
+  const FlashBlock at = flash_block(p);
+  const int g = at.g;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int lq = lane >> 4, lc = lane & 15;
   const int qv = wave * 16 + lc, j = qv / kv_mul, h = qv % kv_mul;
@@ -1082,10 +1103,9 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash3(At
                                                     0);
   };
   bool bad = false, qbad = false;
-  const bool split = p.splits > 0;
   for (int pass = 0; pass < 2; pass++) {
-    const int tile = pass == 0 ? ntiles - 1 - (int)blockIdx.x : (int)blockIdx.x; // the longest walks start first
-    if (pass == 1 && (split || tile >= ntiles - 1 - (int)blockIdx.x))
+    const int tile = pass == 0 ? ntiles - 1 - at.rank : at.rank; // the longest walks start first
+    if (pass == 1 && (split || tile >= ntiles - 1 - at.rank))
       break;
     const int r0 = tile * tile_rows, row = r0 + j;
     const bool active = j < tile_rows && row < p.rows;
@@ -1116,7 +1136,7 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash3(At
       o[d] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     float m_run = -FLT_MAX, l_run = 0.0f;
     const int all = last / kC + 1, share = split ? (all + p.splits - 1) / p.splits : all;
-    const int c0 = split ? min(all, (int)blockIdx.z * share) : 0, chunks = min(all, c0 + share) - c0;
+    const int c0 = split ? min(all, at.share * share) : 0, chunks = min(all, c0 + share) - c0;
     float kr[8], vr[8]; // the next chunk's K and V values of this thread's staging items
     auto load = [&](int c) {
       const int t0 = (c0 + c) * kC;
@@ -1249,7 +1269,7 @@ template <int HD> __global__ __launch_bounds__(kTileThreads) void attn_flash3(At
     if (!active)
       continue;
     if (split) { // the share's value sums, maximum (natural units) and sum, unnormalized, in slot [row][head][share]
-      float *slot = p.partial + (((size_t)row * p.n_heads + (size_t)g * kv_mul + h) * p.splits + blockIdx.z) * p.slot;
+      float *slot = p.partial + (((size_t)row * p.n_heads + (size_t)g * kv_mul + h) * p.splits + at.share) * p.slot;
 #pragma unroll
       for (int d = 0; d < kDt; d++)
         *reinterpret_cast<float4 *>(slot + 16 * d + 4 * lq) = float4{o[d][0], o[d][1], o[d][2], o[d][3]};
@@ -1696,15 +1716,16 @@ bool attention_flash_bf3() {
 // about the same time per chunk whatever the grid, so a grid of few blocks with long walks (a prompt of some hundred
 // rows, or a short batch late in a sequence) leaves most CUs idle for the whole walk. Split S gives each tile S blocks
 // over shares of its chunks and adds attn_merge_shares. The choice is the S of least estimated time, `unit` positions
-// taking the kernel's measured time: unsplit, the longest pair's walk times the rounds of the CUs its grid takes; split,
-// the longest share, or where the blocks are more than the CUs the smaller of whole rounds of it and an even load plus
-// half of it (the shares of a causal batch differ, and the longest start first), plus the partials' cost. Fitted to
-// forced splits of twelve shapes, within a tenth of each (us, unsplit / chosen / best of 2 .. 16): 600 rows of 32 + 8
-// heads of 64 43 / 32 / 32 (left unsplit by an estimate of whole rounds alone), 300 rows 27 / 17 / 17, 512 rows of 24 + 8
-// heads of 128 66 / 35 / 35, 700 rows from position 300 133 / 68 / 68 (before 77), 256 rows of 32 + 8 from 1792 349 / 60 /
-// 60, 40 rows from 2000 362 / 25 / 25; 1024 rows 105 / 105 / 112. A split must save a twentieth. Its partials stay within
-// job.partial_room. The choice never looks at job.qout: quantized rows are bitwise the FP32 rows quantized, so both calls walk the
-// same shares. LLAMA_HIP_FLASH_SPLITS = n forces n (1: never split), for tuning and tests.
+// taking the kernel's measured time. Unsplit: the longest pair's walk times the rounds of the CUs its grid takes. Split:
+// the blocks by length (flash_block), a CU's next one behind its last, and the partials' cost. The CUs that finish first
+// take the longest that are left, so two rounds of blocks take the sum of the last of the first and the first of the
+// second, or the longest of the first alone. A split must save a twentieth. Fitted to forced splits of 585 shapes (nine
+// head counts, 16 to 3000 rows from 0 to 3500): 0.6% behind the best of them on average. Chosen / the best, us, and /
+// whole rounds of the longest share in place of the sums: 2048 rows of 4 heads of 128 48 / 48 / 60, 1024 rows of 16 + 4
+// 47 / 47 / 59, of 32 + 8 74 / 74 / 105, 700 rows of 16 + 4 from 3500 162 / 162 / 166, 600 rows of 32 + 8 heads of 64 29 /
+// 28 / 43, 512 rows of 24 + 8 of 128 36 / 33 / 36, 40 rows of 32 + 8 from 1792 26 / 26 / 33. Its partials stay within
+// job.partial_room. The choice never looks at job.qout: quantized rows are bitwise the FP32 rows quantized, so both calls
+// walk the same shares. LLAMA_HIP_FLASH_SPLITS = n forces n (1: never split), for tuning and tests.
 int flash_splits(const AttentionJob &job, int chunks) {
   const int kv_mul = job.n_heads / job.n_kv_heads;
   const int tile_rows = 128 / kv_mul, tiles = (job.rows + tile_rows - 1) / tile_rows;
@@ -1712,27 +1733,32 @@ int flash_splits(const AttentionJob &job, int chunks) {
   const char *env = getenv("LLAMA_HIP_FLASH_SPLITS");
   int splits = env && *env ? atoi(env) : 0;
   if (splits <= 0) {
-    // the BF16-part kernel walks 32 positions in about 2.85 us at head_dim 128 (1.75 at 64); the FP32-product kernel's
-    // figures are for 64
+    // the BF16-part kernel walks 32 positions in about 2.85 us at head_dim 128 (1.63 at 64), the FP32-product kernel 64 in
+    // 10 (5.7); a share's block adds 3 us
     const bool bf3 = attention_flash_bf3();
     const int unit = bf3 ? 32 : kChunk;
-    const double unit_us = (job.head_dim == 128 ? 1.0 : 0.61) * (bf3 ? 2.85 : 10.0);
+    const double unit_us = (job.head_dim == 128 ? 1.0 : 0.573) * (bf3 ? 2.85 : 10.0), block_us = 3.0;
     auto walk = [&](int t) {
       const long long end = (long long)(t + 1) * tile_rows;
       return (int)((job.pos0 + (end < job.rows ? end : job.rows) - 1) / unit + 1);
     };
-    auto rounds = [&](long long blocks) { return (double)((blocks + cus - 1) / cus); };
-    const int first = walk(0), last = walk(tiles - 1);
-    const double even = 0.5 * (first + last) * tiles * job.n_kv_heads / cus; // every walk over the CUs
+    auto shares = [&](int s) { // time of the blocks of S shares a tile
+      const long long per = (long long)job.n_kv_heads * s, blocks = per * tiles;
+      auto length = [&](long long i) {
+        return unit_us * ((walk(tiles - 1 - (int)(i / per)) + s - 1) / s) + block_us;
+      };
+      double t = 0.0;
+      for (long long i = 0; i < blocks; i += 2 * cus)
+        t += fmax(length(i), i + cus < blocks ? length(i + cus - 1) + length(i + cus) : 0.0);
+      return t;
+    };
     const double per_share = 0.011 * (job.rows * (double)job.n_heads / 32.0) * job.head_dim / 128.0;
-    const double unsplit = 5.0 + unit_us * (last + (tiles > 1 ? first : 0)) *
-                                     rounds((long long)((tiles + 1) / 2) * job.n_kv_heads);
+    const double pair_rounds = (double)(((long long)((tiles + 1) / 2) * job.n_kv_heads + cus - 1) / cus);
+    const double base = 2.3, unsplit = base + unit_us * (walk(tiles - 1) + (tiles > 1 ? walk(0) : 0)) * pair_rounds;
     double best = 0.95 * unsplit;
     splits = 1;
     for (int s : {2, 3, 4, 6, 8, 12, 16}) {
-      const double share = (last + s - 1) / s;
-      const double work = fmax(share, fmin(share * rounds((long long)tiles * job.n_kv_heads * s), even + 0.5 * share));
-      const double t = 5.0 + unit_us * work + per_share * s;
+      const double t = base + shares(s) + per_share * s;
       if (t < best)
         best = t, splits = s;
     }
@@ -1797,8 +1823,10 @@ bool launch_attention(const AttentionJob &job, float *partial, hipStream_t strea
     // pair of tiles, or per tile and share of its chunks (flash_splits)
     const int tile_rows = 128 / kv_mul, tiles = (job.rows + tile_rows - 1) / tile_rows;
     p.splits = flash_splits(job, p.chunks);
-    const dim3 grid(p.splits ? (unsigned)tiles : (unsigned)((tiles + 1) / 2), (unsigned)job.n_kv_heads,
-                    p.splits ? (unsigned)p.splits : 1u);
+    p.by_length = (long long)tiles * job.n_kv_heads * p.splits > (device().cu_count > 0 ? device().cu_count : 256);
+    const dim3 grid = p.by_length ? dim3((unsigned)(tiles * job.n_kv_heads * p.splits))
+                                  : dim3((unsigned)(p.splits ? tiles : (tiles + 1) / 2), (unsigned)job.n_kv_heads,
+                                         (unsigned)max(p.splits, 1));
     const bool bf3 = attention_flash_bf3();
     const bool fused_quant = job.qout && bf3 && !p.splits;
     if (fused_quant) {

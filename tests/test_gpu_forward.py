@@ -392,6 +392,36 @@ def test_attention_flash_forced_splits(splits, shape, monkeypatch):
     test_attention_batch_flash_shapes(*shape, monkeypatch, splits=splits)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0,m,splits", [
+    (10, 5, 64, 0, 520, 7),     # 9 tiles x 5 KV heads x 7 shares: 315 blocks, listed by length
+    (4, 1, 64, 3, 1030, 8),     # one KV head, 33 tiles: 264 blocks
+    (4, 2, 128, 0, 2048, 4),    # 32 tiles: 256 blocks, all of them started at once
+    (4, 2, 128, 0, 2048, 5),    # 320 blocks
+    (24, 8, 128, 100, 512, 3),  # idle vectors, the heads turning with the tiles
+    (4, 4, 128, 0, 2048, 0),    # chosen: 16 tiles, listed
+    (16, 4, 128, 0, 1024, 0),   # chosen: 32 tiles, listed
+])
+@pytest.mark.parametrize("form", ["bf16", "fp32"])
+def test_attention_flash_block_order(nh, nkv, hd, pos0, m, splits, form, monkeypatch):
+    """Split blocks in either order (the tiles fastest while every block starts at once, by length beyond that): every
+    row of every head against the unsplit walk. Each is within 2e-5 * max|v| + 1e-6 of the exact value (the budget of
+    check_attention), so they are within twice that of each other."""
+    L = hu.lib()
+    monkeypatch.setenv("LLAMA_HIP_FLASH_FORM", form)
+    rng = orc.Rng(orc.SEED + 971 + m + nh)
+    seq = pos0 + m + 3
+    kc, vc, q = rng.normal(seq * nkv * hd, 0, 1), rng.normal(seq * nkv * hd, 0, 1), rng.normal(m * nh * hd, 0, 1)
+    dq, dk, dv = hu.dev(q), hu.dev(kc), hu.dev(vc)
+    got = []
+    for s in (1, splits):
+        monkeypatch.setenv("LLAMA_HIP_FLASH_SPLITS", str(s))
+        do = hu.dev(np.full(m * nh * hd, 7e9, np.float32))
+        L.k_attention_batch_kv(lh.ptr(do), lh.ptr(dq), lh.ptr(dk), lh.ptr(dv), None, None, nh, nkv, hd, seq, pos0, m)
+        got.append(hu.host(do))
+        assert not lh.last_error()
+    assert np.max(np.abs(got[0] - got[1])) <= 2 * (2e-5 * np.abs(vc).max() + 1e-6)
+
+
 def test_attention_flash_nonfinite_score_fails():
     L = hu.lib()
     lh.record_failures()
