@@ -2624,8 +2624,14 @@ bool launch_q8_gemm_swiglu_quantized(const GemmQ8Job &job, hipStream_t stream) {
   q8_wide_grid(p, list);
   if (p.sk.splits != 1 || p.grid.total <= 0)
     return false;
-  GemmSegmentDev head, tail;
-  if (q8_wide_tail(p, job.seg[0], head, tail)) { // a partial last round: its columns on the 256 x 128 kernel
+  // A partial last round: its columns on the 256 x 128 kernel. Where the FP32 call does so and the quantized epilogue, which
+  // has no split form, cannot, the rows would not be bitwise the FP32 rows quantized: declined.
+  GemmSegmentDev head, tail, plain = job.seg[0];
+  plain.cq = nullptr;
+  const bool has_tail = q8_wide_tail(p, plain, head, tail);
+  if (has_tail && !q8_wide_tail(p, job.seg[0], head, tail))
+    return false;
+  if (has_tail) {
     q8_wide_grid(p, SegList{&head, 1});
     if (!q8_wide_kernel(p, false, (unsigned)p.grid.total, stream))
       return false;

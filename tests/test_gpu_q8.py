@@ -697,6 +697,42 @@ def test_gemm_q8_swiglu_quantized(m, n, k):
         L.llhip_set_gemm_splits(0)
 
 
+@pytest.mark.parametrize("m,n,ran", [(512, 18432, 0), (512, 20480, 0), (300, 24576, 1), (512, 28672, 1), (700, 14336, 1)])
+@pytest.mark.parametrize("splits", [0, 1])
+def test_gemm_q8_swiglu_quantized_last_round(m, n, ran, splits):
+    """Wide grids with a last round of 32 and 64 (k_gemm_q8 gives it to the narrow kernel, in blocks that may split K: the
+    quantizing call declines and writes nothing), 128 (a whole round of narrow tiles, also at 300 rows) and 192 or 80 of
+    256 CUs (three row tiles: not whole columns; the grid stays whole): where it runs, bitwise k_gemm_q8 then
+    k_quantize_rows."""
+    L, k, gs = hu.lib(), 128, 64
+    if L.llhip_device_cu_count() != 256:
+        pytest.skip("last rounds counted for 256 CUs")
+    xq, xs, wq, ws, w3q, w3s, rng = gemm_case(m, n, k, gs, 6262 + m + n)
+    t = hu.torch()
+    dx = [hu.dev(a) for a in (xq, xs, wq, ws, w3q, w3s)]
+    w1, w3 = lh.w8(dx[2], dx[3]), lh.w8(dx[4], dx[5])
+    try:
+        L.llhip_set_q8_tile(2)
+        L.llhip_set_gemm_splits(splits)
+        hq, hs = hu.dev(np.full((m, n), 7, np.int8)), hu.empty((m, n // 64), t.float32)
+        assert L.llhip_gemm_q8_swiglu_quantize(lh.ptr(dx[0]), lh.ptr(dx[1]), m, k, gs, ctypes.byref(w1), ctypes.byref(w3),
+                                               n, lh.ptr(hq), lh.ptr(hs)) == ran
+        if not ran:
+            assert np.all(hu.host(hq) == 7)
+            return
+        hb = hu.empty((m, n), t.float32)
+        seg = lh.GemmQ8Segment(lh.ptr(hb), n, w1, w3, None, None, n, lh.GEMM_SWIGLU)
+        L.k_gemm_q8(lh.ptr(dx[0]), lh.ptr(dx[1]), m, k, gs, seg, 1)
+        q2, s2 = hu.empty((m, n), t.int8), hu.empty((m, n // 64), t.float32)
+        L.k_quantize_rows(lh.ptr(q2), lh.ptr(s2), lh.ptr(hb), n, m, n, gs)
+        assert lh.last_error() == "", lh.last_error()
+        assert np.array_equal(hu.host(hq), hu.host(q2)), "quantized values"
+        assert np.array_equal(hu.bits(hu.host(hs)), hu.bits(hu.host(s2))), "scales"
+    finally:
+        L.llhip_set_q8_tile(0)
+        L.llhip_set_gemm_splits(0)
+
+
 def test_gemm_q8_qkv_segments_and_gemv_agreement():
     """Three segments sharing the activations (QKV), and each GEMM row against the GEMV of that row."""
     L = hu.lib()
