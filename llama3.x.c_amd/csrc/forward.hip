@@ -185,46 +185,50 @@ __global__ __launch_bounds__(kThreads) void rope_kv_rows(float *__restrict__ q, 
 }
 
 // rope_kv_rows for head_dim HD = 64 or 128: thread (row, d4) of a unit takes dimensions 4 d4 .. 4 d4 + 3 of two q heads
-// of its row, or of one KV head (k and v), its loads in flight together and the row's table values loaded once for
-// them. Each element gets the same products in the same order as in rope_kv_rows, so the results are bitwise those of
-// rope_kv_rows. Latency bounds it until the rows are many, then the memory: 2 rows of 32 + 8 heads of 128 take 2.4 us,
-// 256 rows 4.1 us (3.4 TB/s) and 2048 rows 19.9 us (5.5 TB/s) where a thread that walked every head of its row, each
-// load behind the one before, took 7.7, 10.1 and 20.4 us. A block's neighbours take the next heads of the same rows,
-// not the next rows of the same heads: the latter, a row's stride apart, ran 256 rows in 12 us.
-template <int HD>
+// of its row, or of one KV head (k and v), its loads in flight together; WALK: of every unit of its row in turn. Each
+// element gets the same products in the same order as in rope_kv_rows, so the results are bitwise those of rope_kv_rows.
+// Latency bounds it until the rows are many, then the memory. A thread a unit is the faster form until the rows alone
+// have a block for every CU: 2 rows of 32 + 8 heads of 128 2.4 us (walked 7.7), 256 rows 4.3 (9.1; 3.4 TB/s), 1500 rows of
+// 24 + 8 13.5 (14.5). From there the walk, whose blocks stream whole rows, is: 2048 rows 16.8 (17.6), 4096 rows 28.4
+// (32.6; 5.8 TB/s), of 64 dimensions 8192 rows of 32 + 8 33.6 (37.4), 4096 rows 21.2 (20.1). A block's neighbours take the
+// next units of the same rows, not the next rows of the same units: the latter, a row's stride apart, ran 256 rows in 12
+// us.
+template <int HD, bool WALK>
 __global__ __launch_bounds__(kThreads) void rope_kv_rows_hd(float *__restrict__ q, size_t q_stride, float *__restrict__ k,
                                                             const float *__restrict__ v, size_t kv_stride,
-                                                            const float *__restrict__ table, size_t table_stride,
-                                                            int rows, int n_heads, int n_kv_heads,
-                                                            float *__restrict__ key_cache,
+                                                            const float *__restrict__ table, size_t table_stride, int rows,
+                                                            int n_heads, int n_kv_heads, float *__restrict__ key_cache,
                                                             float *__restrict__ value_cache, int pos0,
                                                             size_t pos_stride, size_t head_base) {
   constexpr int hd4 = HD / 4, kRowsPerBlock = kThreads / hd4;
   const int qunits = (n_heads + 1) / 2, units = qunits + n_kv_heads;
-  const int unit = blockIdx.x % units;
-  const int r = blockIdx.x / units * kRowsPerBlock + threadIdx.x / hd4, d = 4 * (threadIdx.x % hd4);
+  int unit = WALK ? 0 : blockIdx.x % units;
+  const int block = WALK ? blockIdx.x : blockIdx.x / units;
+  const int r = block * kRowsPerBlock + threadIdx.x / hd4, d = 4 * (threadIdx.x % hd4);
   if (r >= rows)
     return;
   const float *t = table + (size_t)r * table_stride;
-  if (unit < qunits) {
-    float4 *pq = reinterpret_cast<float4 *>(q + (size_t)r * q_stride + (size_t)(2 * unit) * HD + d);
-    const bool two = 2 * unit + 1 < n_heads;
-    const float4 x0 = pq[0], x1 = pq[two ? hd4 : 0];
-    const Rot4 rot = rot4_of(t, HD, d);
-    pq[0] = rotate4(x0, rot);
-    if (two)
-      pq[hd4] = rotate4(x1, rot);
-    return;
-  }
-  const int g = unit - qunits;
-  const size_t at = (size_t)r * kv_stride + (size_t)g * HD + d;
-  const size_t slot = (size_t)(pos0 + r) * pos_stride + (size_t)g * head_base + d;
-  float4 *pk = reinterpret_cast<float4 *>(k + at);
-  const float4 x = *pk, y = *reinterpret_cast<const float4 *>(v + at);
-  const float4 z = rotate4(x, rot4_of(t, HD, d));
-  *pk = z;
-  *reinterpret_cast<float4 *>(key_cache + slot) = z;
-  *reinterpret_cast<float4 *>(value_cache + slot) = y;
+  do {
+    if (unit < qunits) {
+      float4 *pq = reinterpret_cast<float4 *>(q + (size_t)r * q_stride + (size_t)(2 * unit) * HD + d);
+      const bool two = 2 * unit + 1 < n_heads;
+      const float4 x0 = pq[0], x1 = pq[two ? hd4 : 0];
+      const Rot4 rot = rot4_of(t, HD, d);
+      pq[0] = rotate4(x0, rot);
+      if (two)
+        pq[hd4] = rotate4(x1, rot);
+    } else {
+      const int g = unit - qunits;
+      const size_t at = (size_t)r * kv_stride + (size_t)g * HD + d;
+      const size_t slot = (size_t)(pos0 + r) * pos_stride + (size_t)g * head_base + d;
+      float4 *pk = reinterpret_cast<float4 *>(k + at);
+      const float4 x = *pk, y = *reinterpret_cast<const float4 *>(v + at);
+      const float4 z = rotate4(x, rot4_of(t, HD, d));
+      *pk = z;
+      *reinterpret_cast<float4 *>(key_cache + slot) = z;
+      *reinterpret_cast<float4 *>(value_cache + slot) = y;
+    }
+  } while (WALK && ++unit < units);
 }
 
 // ---- embedding rows -------------------------------------------------------------------------------------------------
@@ -1581,14 +1585,18 @@ bool launch_rope_kv_rows(float *q, size_t q_stride, float *k, const float *v, si
   const int per_row = (n_heads + 2 * n_kv_heads) * (head_dim / 4);
   if (head_dim == 128 || head_dim == 64) {
     const int rows_per_block = kThreads / (head_dim / 4), units = (n_heads + 1) / 2 + n_kv_heads;
-    const int most = max(kMaxBlocks / units, 1) * rows_per_block; // rows of a launch
+    const int cus = device().cu_count > 0 ? device().cu_count : 256;
+    // a block of rows for every CU (for one and a half of them at 64 dimensions): a thread walks its row's units
+    const bool walk = rows / rows_per_block >= (head_dim == 128 ? cus : cus + cus / 2);
+    const int per_rows = walk ? 1 : units, most = max(kMaxBlocks / per_rows, 1) * rows_per_block; // rows of a launch
+    const auto kernel = head_dim == 128 ? (walk ? rope_kv_rows_hd<128, true> : rope_kv_rows_hd<128, false>)
+                                        : (walk ? rope_kv_rows_hd<64, true> : rope_kv_rows_hd<64, false>);
     for (int r0 = 0; r0 < rows; r0 += most) {
       const int n = min(most, rows - r0);
-      const dim3 grid((unsigned)((n + rows_per_block - 1) / rows_per_block) * (unsigned)units);
-      hipLaunchKernelGGL(head_dim == 128 ? rope_kv_rows_hd<128> : rope_kv_rows_hd<64>, grid, dim3(kThreads), 0, stream,
-                         q + (size_t)r0 * q_stride, q_stride, k + (size_t)r0 * kv_stride, v + (size_t)r0 * kv_stride,
-                         kv_stride, table + (size_t)r0 * table_stride, table_stride, n, n_heads, n_kv_heads, key_cache,
-                         value_cache, pos0 + r0, pos_stride, head_base);
+      const dim3 grid((unsigned)((n + rows_per_block - 1) / rows_per_block) * (unsigned)per_rows);
+      hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, q + (size_t)r0 * q_stride, q_stride,
+                         k + (size_t)r0 * kv_stride, v + (size_t)r0 * kv_stride, kv_stride, table + (size_t)r0 * table_stride,
+                         table_stride, n, n_heads, n_kv_heads, key_cache, value_cache, pos0 + r0, pos_stride, head_base);
       if (rows - r0 <= most)
         break;
     }

@@ -662,10 +662,12 @@ def test_rope_kv_store_rows_fused(rows, nh, nkv, hd, seq, pos0, layout):
         L.kernels_kv_layout_select(b"head")
 
 
-@pytest.mark.parametrize("rows,nh,nkv,hd", [(1, 1, 1, 128), (7, 3, 3, 128), (8, 5, 1, 128), (9, 2, 2, 64), (17, 15, 3, 64)])
+@pytest.mark.parametrize("rows,nh,nkv,hd", [(1, 1, 1, 128), (7, 3, 3, 128), (8, 5, 1, 128), (9, 2, 2, 64), (17, 15, 3, 64),
+                                            (2047, 3, 1, 128), (2049, 3, 2, 128), (6143, 1, 1, 64), (6145, 3, 2, 64)])
 def test_rope_kv_store_rows_head_counts(rows, nh, nkv, hd):
-    """The rows kernel of head_dim 64 and 128 takes two q heads or one KV head per unit: odd head counts, and rows on
-    both sides of a block's 8 or 16, bitwise the separate calls; the rows of the strides' padding stay untouched."""
+    """The rows kernel of head_dim 64 and 128 takes two q heads or one KV head per unit: odd head counts, rows on both
+    sides of a block's 8 or 16 and of the line where a thread walks its row's units (2048 rows, 6144 of 64), bitwise the
+    separate calls; the rows of the strides' padding stay untouched."""
     L = hu.lib()
     rng = orc.Rng(orc.SEED + 4700 + rows + nh + hd)
     qs, ks, seq, pos0 = nh * hd + 8, nkv * hd + 4, rows + 5, 3
