@@ -251,9 +251,9 @@ __global__ __launch_bounds__(kThreads) void embed_rows(float *__restrict__ out, 
   out[(size_t)r * dim + j] = (float)table[at] * scales[at / gs];
 }
 
-// The same for dim and gs multiples of 4 and aligned operands: four values of one scale per thread, per_row blocks a
-// row. The write of the rows bounds it: 2048 ids of 4096 values take 9.3 us (4.5 TB/s), where one value a thread behind
-// two 64-bit divisions took 20.6 us; 256 ids 3.2 us, before 4.2.
+// The same for dim and gs multiples of 4, at least 256 values and aligned operands: four values of one scale per thread,
+// per_row blocks a row. The write of the rows bounds it: 2048 ids of 4096 values take 9.3 us (4.5 TB/s), where one value a
+// thread behind two 64-bit divisions took 20.6 us; 256 ids 3.2 us, before 4.2.
 __global__ __launch_bounds__(kThreads) void embed_rows4(float *__restrict__ out, const int8_t *__restrict__ table,
                                                         const float *__restrict__ scales, const int *__restrict__ ids,
                                                         unsigned per_row, unsigned dim, unsigned gs, int vocab,
@@ -1620,7 +1620,9 @@ bool launch_kv_store(float *cache, const float *src, size_t src_ld, int pos0, in
 bool launch_embed_rows(float *out, const int8_t *table, const float *scales, const int *ids, int count, int dim,
                        int gs, int vocab, hipStream_t stream) {
   const long long per_row = ((long long)dim + 4 * kThreads - 1) / (4 * kThreads);
-  if (dim % 4 == 0 && gs % 4 == 0 && ((uintptr_t)table & 3) == 0 && ((uintptr_t)out & 15) == 0 &&
+  // rows of fewer than 256 values leave three quarters of a row's block idle: 2048 ids of 96 values 3.1 us, one value a
+  // thread 2.8
+  if (dim % 4 == 0 && gs % 4 == 0 && dim >= kThreads && ((uintptr_t)table & 3) == 0 && ((uintptr_t)out & 15) == 0 &&
       count * per_row <= kMaxBlocks) {
     hipLaunchKernelGGL(embed_rows4, dim3((unsigned)(count * per_row)), dim3(kThreads), 0, stream, out, table, scales, ids,
                        (unsigned)per_row, (unsigned)dim, (unsigned)gs, vocab, device().error_flags);

@@ -481,12 +481,12 @@ def test_attention_nonfinite_score_fails_and_bookkeeping():
 # ---- embedding rows ------------------------------------------------------------------------------------------------
 
 
-@pytest.mark.parametrize("dim,gs,shift", [(4, 4, 0), (1020, 60, 0), (1024, 64, 0), (1028, 4, 0), (2176, 128, 0),
-                                          (1026, 6, 0), (1024, 64, 1)])
+@pytest.mark.parametrize("dim,gs,shift", [(4, 4, 0), (252, 4, 0), (256, 64, 0), (1020, 60, 0), (1024, 64, 0), (1028, 4, 0),
+                                          (2176, 128, 0), (1026, 6, 0), (1024, 64, 1)])
 def test_embed_q8_rows_widths(dim, gs, shift):
     """Widths on both sides of the 1024 values that a block of four values a thread takes, groups that fill rows and
-    that straddle them, and the one-value kernel (a dim that is no multiple of 4, a table at an odd address): bitwise
-    numpy's float32 product."""
+    that straddle them, and the one-value kernel (fewer than 256 values, a dim that is no multiple of 4, a table at an odd
+    address): bitwise numpy's float32 product."""
     L = hu.lib()
     rng = np.random.default_rng(orc.SEED + 911 + dim + gs)
     vocab = 2 * gs
