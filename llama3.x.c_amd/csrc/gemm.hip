@@ -1154,16 +1154,16 @@ __global__ __launch_bounds__(kQ8Threads, 2) void mm_gemm_lds(MmParams p) {
 // Delivery of the operands bounds the BF16 tiles, not the MFMAs (a copy of a kernel with 64-byte steps and five stages
 // took the same time without its MFMAs): a row's 64 bytes of A are half a cache line, so each step fetched the line of
 // the step before again. Here a stage takes two steps, 128 bytes of each row, as eight rows per 1 KB load; three stages
-// of 48 KB hold as many steps in flight. A row's eight 16-byte chunks lie at chunk ^ (row % 8), so the operand reads of
-// eight consecutive rows fall on distinct banks. Measured, 64-byte steps / this (us, the panel's rounding included): 512
-// x 2 * 8192 x 3072 SwiGLU 71 / 58 (880 TFLOP/s), 512 x 3072 x 8192 56 / 50, 512 x 5120 x 3072 41 / 37, 2048 x 3072 x
-// 8192 195 / 158 (650 TFLOP/s). Without its loads the SwiGLU shape takes 50: LDS reads and MFMAs, 1.2 PFLOP/s, the rate
-// a library product of 8192 cubed reaches here.
+// of 48 KB hold as many steps in flight. The reads that reach L2 fall by 39% (512 x 2 * 8192 x 3072 SwiGLU 7.7 to 4.7
+// million), with the same misses there. A row's eight 16-byte chunks lie at chunk ^ (row % 8), so the operand reads of
+// eight consecutive rows fall on distinct banks (no bank conflict counted). Measured, 64-byte steps / this (us, the
+// panel's rounding included): 512 x 2 * 8192 x 3072 SwiGLU 58 / 53.5 (960 TFLOP/s), 512 x 3072 x 8192 46 / 42, 512 x 3072
+// x 3072 31 / 28, 2048 x 3072 x 8192 123 / 114 (900 TFLOP/s).
 // The same tile and stage shapes serve the FP32 form on BF16 parts (a stage holds 32 FP32 values of each row). MI is
 // the wave's 16-row MFMA tiles: 256, 192, 128 or 64 rows a block, the fewest that hold the batch in as many row tiles
 // as 256-row blocks take, with more stages where the rows are few and the weights' latency is what there is to hide
-// (BF16, 256-row tiles / this: 20 x 2 * 8192 x 2048 31 / 21 us, 20 x 2048 x 8192 26 / 19, 180 x 4096 x 4096 28 / 26, 300
-// x 4096 x 14336 74 / 64).
+// (BF16, 256-row tiles of 64-byte steps / this: 20 x 2 * 8192 x 2048 28 / 20 us, 20 x 2048 x 8192 40 / 18, 180 x 4096 x
+// 4096 33.5 / 23.5, 300 x 4096 x 14336 65 / 55).
 template <int MI_, int STAGES_> struct MmCfg {
   static constexpr int MI = MI_, Stages = STAGES_, TileM = 64 * MI;
   static constexpr int Loads = MI + 2;                        // per wave and stage: MI blocks of A and two of B
@@ -1266,14 +1266,16 @@ template <class C> __global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_ld
 
   // The pair in stage ST: its first step's MFMAs (operands already in registers) while the second step's are read;
   // then every wave is done with the stage once its reads are, the next pair has landed once only those after it may be
-  // outstanding, and the pair Stages further fills the stage while the second step's MFMAs run.
+  // outstanding, and the pair Stages further fills the stage while the second step's MFMAs run. The compiler spreads a
+  // step's operand reads over the other step's MFMAs: with a fence that kept them in front, a wave issued no MFMA behind
+  // the barrier until all of them were on their way (fenced / this, us: 700 x 6144 x 4096 66 / 58.5, 700 x 4096 x 14336 112 /
+  // 101, 2048 x 3072 x 8192 125 / 114; with 64-byte steps and five stages 61, 107 and 123).
   constexpr std::integral_constant<int, 0> first{};
   constexpr std::integral_constant<int, 1> second{};
   Operands cur, next;
   auto advance = [&](int step, auto ST) {
     constexpr int nst = (decltype(ST)::value + 1) % C::Stages;
     operands(ST, second, next);
-    __builtin_amdgcn_sched_barrier(0);
     mfmas(cur);
     __builtin_amdgcn_sched_barrier(0);
     cur = next;
@@ -1281,7 +1283,6 @@ template <class C> __global__ __launch_bounds__(kQ8Threads, 2) void bf16_gemm_ld
     __builtin_amdgcn_s_barrier();
     issue(step + 2 * C::Stages, ST);
     operands(std::integral_constant<int, nst>{}, first, next);
-    __builtin_amdgcn_sched_barrier(0);
     mfmas(cur);
     __builtin_amdgcn_sched_barrier(0);
     cur = next;
