@@ -770,10 +770,10 @@ __global__ __launch_bounds__(C::Threads, 2) void q8_gemm_lds(Q8Params p) {
 // q8_gemm_lds's tile and arithmetic (the same expression in the same group order: unsplit, bit for bit its results) with
 // the row tiles and 128-byte stages of bf16_gemm_lds: a stage holds two groups, 128 bytes of each row, and a block 192,
 // 128 or 64 rows by the batch, with more stages where the rows are few. A row's 128 bytes are one whole cache line where
-// the block's K range begins at an even group; a split's range may begin at an odd one, and its lines then hold half of
-// two stages each. In 256-row tiles the rows past the batch cost their share of the MFMAs and the rescale all the same.
-// Measured, q8_gemm_lds / this (us): 40 x 2 * 14336 x 4096 SwiGLU 65 / 44, 40 x 4096 x 14336 43 / 29, 100 x 2048 x 8192
-// 26 / 21, 128 x 3072 x 3072 26 / 20, 333 x 2 * 8192 x 3072 59 / 52.
+// K is a multiple of 128: a split's range begins at an even group (in ranges that began at any, 600 x 2048 x 8192 38.7 us,
+// so 37.0, 180 x 6144 x 4096 27.8 / 26.9). In 256-row tiles the rows past the batch cost their share of the MFMAs and the
+// rescale all the same. Measured, q8_gemm_lds / this (us): 40 x 2 * 14336 x 4096 SwiGLU 65 / 44, 40 x 4096 x 14336 43 / 29,
+// 100 x 2048 x 8192 26 / 21, 128 x 3072 x 3072 26 / 20, 333 x 2 * 8192 x 3072 59 / 52.
 // 256-row tiles stay with q8_gemm_lds. A form of this kernel for them halved the loads that reach L2 (2048 x 3072 x 8192:
 // 18.8 to 10.0 million) but waits at its barrier for the operands it reads right behind it (waves' waiting cycles 24 to
 // 32 million): 2048 x 3072 x 8192 125 / 134 us, 1024 x 6144 x 4096 68 / 73, 256 x 2 * 14336 x 4096 72 / 74, 3 to 8% slower
@@ -2344,7 +2344,8 @@ template <int MI> bool q8_rows_launch(Q8Params p, const SegList &segs, hipStream
   if (p.grid.total <= 0)
     return true;
   const int steps = p.k / 64;
-  p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, steps, &p.sk.per);
+  const int unit = forced_splits.load() > 0 ? 1 : 2; // whole stages; a forced count gives every tiling the same K ranges
+  p.sk.splits = p.grid.total > kSplitSlots ? 1 : choose_splits(p.grid.total, steps, &p.sk.per, unit);
   p.sk.partial = (v4f *)device().split_partial;
   p.sk.count = device().split_count;
   if (p.sk.splits == 1) {
@@ -2372,7 +2373,7 @@ int q8_tile_height(const Q8Params &p, const SegList &segs) {
     static const double group_us[4] = {0.52, 0.72, 0.97, 1.25};
     const int tiles = make_q8_grid(segs.seg, segs.nseg, p.m, 64 * mi).total;
     int per = steps;
-    const int splits = tiles > kSplitSlots ? 1 : choose_splits(tiles, steps, &per);
+    const int splits = tiles > kSplitSlots ? 1 : choose_splits(tiles, steps, &per, 2);
     const int blocks = tiles * splits;
     return (double)((blocks + cus - 1) / cus) * (splits > 1 ? per : steps) * group_us[mi - 1] +
            (splits > 1 ? 6.0 + blocks * mi * 32.768e-3 / 2.5 : 3.0);
