@@ -103,9 +103,9 @@ void llhip_set_gemv_shape(int waves_per_row, int blocks_per_cu, int block_waves)
  * most 32 rows to the tiled kernel instead of the weight-streaming one. For tuning and tests. */
 void llhip_set_gemm_splits(int splits);
 
-/* Output tile of the BF16 prefill GEMM: 1 = 256 x 128, 2 = 256 x 256, 0 = by grid (256 x 256 when the grid has at
- * least four 256 x 128 tiles per CU; LLAMA_HIP_BF16_TILE=narrow|wide sets the same at start-up). Results do not depend
- * on it beyond FP32 summation order. For tuning and tests. */
+/* Output tile of the BF16 prefill GEMM: 1 = 256 x 128 (or fewer rows, by the batch), 2 = 256 x 256, 0 = by grid (256 x 256
+ * where its rounds of one tile per CU, weighted 1.7, are fewer; LLAMA_HIP_BF16_TILE=narrow|wide sets the same at
+ * start-up). Results do not depend on it beyond FP32 summation order. For tuning and tests. */
 void llhip_set_bf16_tile(int tile);
 
 /* Output tile of the INT8 prefill GEMM with gs = 64: 1 = 256 x 128, 2 = 256 x 256, 0 = by grid (256 x 256 when the

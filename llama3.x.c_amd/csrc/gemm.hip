@@ -2800,13 +2800,16 @@ bool wide_launch(MmParams p, const GemmF32Job &job, hipStream_t stream) {
   return launch_split_reduce<8, kQ8Threads>(p.grid, p.sk, p.m, kWTileM, kWTileN, stream);
 }
 
-// BF16 tile: LLAMA_HIP_BF16_TILE = wide (256 x 256) or narrow (256 x 128), read once; by default wide when the grid
-// has at least four 256 x 128 tiles per CU. Measured: 2048 x 28672 x 4096 SwiGLU 886 TF/s wide, 754 narrow; with fewer
-// tiles the wide grid's quantization and split cost more than its operand savings (2048 x 4096 x 4096: 677 vs 757,
-// the 512-token 3B shapes 10-15% slower).
+// BF16 tile: LLAMA_HIP_BF16_TILE = wide (256 x 256) or narrow (256 x 128, or fewer rows), read once; by default by rounds
+// of one tile per CU, a wide tile's weighted 1.7 and a narrow one's by its share of 256 rows. Measured narrow / wide (us;
+// rounds of each): 2048 x 2 * 14336 x 4096 466 / 450 (7, 4), 1024 x 2 * 14336 x 4096 251 / 227 (4, 2), 512 x 2 * 14336 x
+// 4096 127 / 115, 2048 x 6144 x 4096 121 / 106 and 1024 x 2 * 8192 x 3072 103 / 94 (2, 1); 1536 x 2 * 8192 x 3072 151 / 164
+// and 3000 x 6144 x 4096 185 / 209 (3, 2), 2048 x 4096 x 4096 75 / 88, 2048 x 4096 x 14336 234 / 243 and 512 x 2 * 8192 x
+// 3072 53 / 68 (1, 1); with lower tiles, 300 x 2 * 14336 x 4096 93 / 102 (192 rows; 2, 1), 513 x 128256 x 2048 340 / 353
+// (192 rows; 12, 6), 128 x 128256 x 2048 128 / 128 (128 rows; 4, 2).
 std::atomic<int> forced_bf16_tile{0}; // llhip_set_bf16_tile: 0 unset, 1 narrow, 2 wide
 
-bool bf16_wide(int narrow_tiles) {
+bool bf16_wide(const GemmF32Job &job, int narrow) {
   static const int env_tile = [] {
     const char *env = getenv("LLAMA_HIP_BF16_TILE");
     return env && !strcmp(env, "wide") ? 2 : env && !strcmp(env, "narrow") ? 1 : 0;
@@ -2815,7 +2818,10 @@ bool bf16_wide(int narrow_tiles) {
   if (forced)
     return forced == 2;
   const int cus = device().cu_count > 0 ? device().cu_count : 256;
-  return narrow_tiles >= 4 * cus;
+  if (narrow < cus)
+    return false;
+  const int wide = make_q8_grid(job.seg, job.nseg, job.m, kWTileM, kWTileN).total;
+  return 17LL * 4 * ((wide + cus - 1) / cus) < 10LL * row_tiles(job.m) * ((narrow + cus - 1) / cus);
 }
 
 bool aligned16(const void *ptr) { return ((uintptr_t)ptr & 15) == 0; }
@@ -2865,7 +2871,7 @@ bool launch_f32_gemm(const GemmF32Job &job, hipStream_t stream) {
     p.a = (const unsigned char *)job.panel;
     p.arow = (long long)kp * 2;
     p.steps = kp / 32;
-    return bf16_wide(p.grid.total) ? wide_launch(p, job, stream) : mm_tiles_launch<false>(p, job, stream);
+    return bf16_wide(job, p.grid.total) ? wide_launch(p, job, stream) : mm_tiles_launch<false>(p, job, stream);
   }
   if (f32_fast_path(job)) {
     p.a = (const unsigned char *)job.a;

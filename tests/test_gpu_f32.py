@@ -443,3 +443,35 @@ def test_gemm_row_tiles(mode, m):
         L.llhip_set_bf16_tile(0)
         if mode == "bf16":
             L.aligned_buffer_free(panel)
+
+
+@pytest.mark.parametrize("m,n,wide", [(512, 16384, 0), (512, 16512, 1), (700, 16384, 1), (513, 16384, 0), (257, 32768, 0),
+                                      (768, 32768, 0), (1024, 32768, 1), (128, 131072, 0)])
+def test_bf16_tile_choice(m, n, wide):
+    """The choice between the 256 x 256 BF16 tiles and the narrow ones (rounds of 256 CUs, wide ones weighted 1.7, narrow
+    ones by their rows): on both sides of it the chosen launch is bit for bit the forced one, and rows of it are within
+    2e-6 * sum|a w| of float64 on the BF16 operands (sums of 32 terms, 2^-24 each)."""
+    L, k = hu.lib(), 32
+    if L.llhip_device_cu_count() != 256:
+        pytest.skip("rounds counted for 256 CUs")
+    rng = orc.Rng(orc.SEED + 173 * m + n)
+    a, w = rng.uniform(m * k, 2.0).reshape(m, k), rng.uniform(n * k).reshape(n, k)
+    pw = np.zeros(L.bf16_vnni_elements(n, k), np.uint16)
+    L.pack_bf16_vnni(lh.ptr(pw), lh.ptr(w), n, k, k)
+    da, dw, dc = hu.dev(a), hu.dev(pw), hu.empty((m, n), hu.torch().float32)
+    panel = lh.AlignedBuffer()
+    L.aligned_buffer_alloc(panel, L.k_gemm_bf16_panel_bytes(m, k), 1)
+    seg = lh.GemmBf16Segment(lh.ptr(dc), n, lh.ptr(dw), None, n, lh.GEMM_STORE)
+    got = []
+    try:
+        for tile in (0, 2 if wide else 1):
+            L.llhip_set_bf16_tile(tile)
+            L.k_gemm_bf16(lh.ptr(da), k, m, k, seg, 1, panel)
+            got.append(hu.host(dc))
+        assert np.array_equal(hu.bits(got[0]), hu.bits(got[1]))
+        rows = [0, 1, m // 2, m - 1]
+        r, mag = ref_f32(bf16_round(a[rows]), bf16_round(w))
+        hu.assert_within_budget(got[0][rows], r, mag, rel=2e-6, what=f"{m}x{n}")
+    finally:
+        L.llhip_set_bf16_tile(0)
+        L.aligned_buffer_free(panel)
