@@ -4,16 +4,18 @@
 // ADD and SWIGLU (a column tile then holds columns of W1 and the same columns of W3, so the gate is applied in
 // registers). The kernels, each described where it is defined:
 //   q8_gemm_lds     int8, 256 x 128 tiles (or 128 x 128), A/B/scales streamed into LDS five stages deep;
-//   q8_gemm_rows    int8 with gs = 64, 64 to 256 rows a tile, two groups a stage;
+//   q8_gemm_rows    int8 with gs = 64, 64 to 192 rows a tile, two groups a stage;
+//   q8_gemm_wide, q8_gemm_wide_smma  int8 with gs = 64, 256 x 256 tiles for large grids;
 //   mm_gemm_lds     FP32, 256 x 128 tiles, the same pipeline;
-//   mm_gemm_f32x3   FP32 on the BF16 matrix cores, the default FP32 kernel;
-//   bf16_gemm_lds   BF16, 256 x 128 tiles, two K steps a stage;
+//   mm_gemm_f32x3   FP32 on the BF16 matrix cores, the default FP32 kernel, 64 to 256 rows a tile, two K steps a stage;
+//   bf16_gemm_lds   BF16, the same tiles and stages;
 //   bf16_gemm_wide  BF16, 256 x 256 tiles for large grids;
-//   split_reduce    the second kernel of a split-K launch of the int8 and wide kernels;
+//   split_reduce    the second kernel of a split-K launch (of an FP32 or narrow BF16 one from four splits);
 //   f32_gemm_mfma   FP32 shapes the pipeline does not take (K % 16 != 0, unaligned rows): 128 x 128 tiles staged
 //                   through registers into double-buffered LDS;
 //   q8_gemm_generic int8 with a group size that is not a multiple of 64.
-// Each wave owns 64 x 64 (64 x 128 in the wide kernel) as a grid of 16 x 16 MFMA tiles. MFMA operand loads are
+// Each wave owns 64 x 64 (64 x 128 in the wide kernels, a quarter of a lower tile's rows x 64) as a grid of 16 x 16 MFMA
+// tiles. MFMA operand loads are
 // symmetric (lane l supplies row l % 16 of A and column l % 16 of W with the same K slice), so the dot products do not
 // depend on how the instruction orders K inside a lane; the 16 x 16 result holds C[4 (l / 16) + e][l % 16] in element
 // e of lane l.
@@ -51,7 +53,7 @@ struct TileSeg {
   int epi;
   int first_tile; // first logical tile of this segment
   int ntiles;     // its column tiles
-  int8_t *cq;     // SWIGLU output quantized in groups of 64 (the wide int8 kernel only), else null
+  int8_t *cq;     // SWIGLU output quantized in groups of 64 (the wide int8 kernels and q8_gemm_lds), else null
   float *cs;
 };
 
@@ -315,7 +317,7 @@ struct Q8Grid {
 constexpr int kSplitSlots = LLHIP_SPLIT_SLOTS; // partial tiles the workspace holds
 
 struct SplitK {
-  v4f *partial;    // [tile * splits + split][16][threads] partial sums, in the accumulators' register order
+  v4f *partial;    // [tile * splits + split][MI * J][threads] partial sums (MI x J MFMA tiles a wave), in register order
   unsigned *count; // [tile] blocks arrived; zero between launches
   int splits;      // blocks per tile (1: no split)
   int per;         // K steps per split
