@@ -1732,8 +1732,8 @@ bool attention_flash_bf3() {
 // second, or the longest of the first alone. A split must save a twentieth. Fitted to forced splits of 585 shapes (nine
 // head counts, 16 to 3000 rows from 0 to 3500): 0.6% behind the best of them on average. Chosen / the best, us, and /
 // whole rounds of the longest share in place of the sums: 2048 rows of 4 heads of 128 48 / 48 / 60, 1024 rows of 16 + 4
-// 47 / 47 / 59, of 32 + 8 74 / 74 / 105, 700 rows of 16 + 4 from 3500 162 / 162 / 166, 600 rows of 32 + 8 heads of 64 29 /
-// 28 / 43, 512 rows of 24 + 8 of 128 36 / 33 / 36, 40 rows of 32 + 8 from 1792 26 / 26 / 33. Its partials stay within
+// 47 / 47 / 58, of 32 + 8 72 / 74 / 105, 700 rows of 16 + 4 from 3500 164 / 165 / 166, 600 rows of 32 + 8 heads of 64 28 /
+// 28 / 43, 512 rows of 24 + 8 of 128 33 / 33 / 36, 40 rows of 32 + 8 from 1792 26 / 26 / 33. Its partials stay within
 // job.partial_room. The choice never looks at job.qout: quantized rows are bitwise the FP32 rows quantized, so both calls
 // walk the same shares. LLAMA_HIP_FLASH_SPLITS = n forces n (1: never split), for tuning and tests.
 int flash_splits(const AttentionJob &job, int chunks) {

@@ -296,7 +296,7 @@ def test_attention_batch_rows(nh, nkv, hd, seq, pos0, m):
     (12, 4, 64, 300, 21, 100, "rows"),     # kv_mul 3, a ragged last tile
     (20, 4, 64, 200, 0, 60, "head"),       # kv_mul 5: 25-row tiles, 3 vectors idle
     (48, 8, 128, 160, 3, 50, "rows"),      # kv_mul 6: 21-row tiles, 2 vectors idle
-    (32, 8, 128, 600, 0, 512, "head"),     # a short 8B prompt: 64 blocks
+    (32, 8, 128, 600, 0, 512, "head"),     # a short 8B prompt: 3 blocks per tile, listed by length
     (24, 8, 128, 700, 40, 512, "rows"),    # the 3B heads from position 40
     (32, 8, 64, 300, 0, 130, "head"),      # 1B heads, 130 rows
     (32, 8, 128, 2100, 1792, 256, "head"), # a 256-row batch late in an 8B prompt: tiles split over 4 blocks each
@@ -308,8 +308,8 @@ def test_attention_batch_flash_shapes(nh, nkv, hd, seq, pos0, m, layout, monkeyp
     """Batches of at least 16 rows with 64 or 128 dimensions per head run the flash kernel (its products from exact
     BF16 parts on the BF16 matrix cores): every checked row within the float64 budget of the decode attention at its position and within twice it of the
     oracle, for GQA ratios 1-16 (those that do not divide 128 leave the tile's last vectors idle), both layouts, ragged
-    tiles, short prompts and long contexts. A short batch late in a sequence splits each tile's positions over several
-    blocks whose partials attn_merge combines (the last four cases, and the 16-row one)."""
+    tiles, short prompts and long contexts. Short prompts and batches late in a sequence split each tile's positions over
+    several blocks whose partials attn_merge_shares combines (all but the 2048-row cases)."""
     if splits:
         monkeypatch.setenv("LLAMA_HIP_FLASH_SPLITS", str(splits))
     L = hu.lib()
