@@ -15,10 +15,9 @@
 //                   through registers into double-buffered LDS;
 //   q8_gemm_generic int8 with a group size that is not a multiple of 64.
 // Each wave owns 64 x 64 (64 x 128 in the wide kernels, a quarter of a lower tile's rows x 64) as a grid of 16 x 16 MFMA
-// tiles. MFMA operand loads are
-// symmetric (lane l supplies row l % 16 of A and column l % 16 of W with the same K slice), so the dot products do not
-// depend on how the instruction orders K inside a lane; the 16 x 16 result holds C[4 (l / 16) + e][l % 16] in element
-// e of lane l.
+// tiles. MFMA operand loads are symmetric (lane l supplies row l % 16 of A and column l % 16 of W with the same K slice),
+// so the dot products do not depend on how the instruction orders K inside a lane; the 16 x 16 result holds
+// C[4 (l / 16) + e][l % 16] in element e of lane l.
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
@@ -2297,8 +2296,8 @@ Q8Grid make_q8_grid(const GemmSegmentDev *segs, int nseg, int m, int tile_m = kQ
   return g;
 }
 
-// 16-row MFMA tiles per wave (a quarter of a block's rows) of the kernels with 64 to 256 rows
-// a tile: the fewest that hold the batch in as many row tiles as 256-row blocks take.
+// 16-row MFMA tiles per wave (a block's rows / 64) of the kernels with 64 to 256 rows a tile: the fewest that hold the batch
+// in as many row tiles as 256-row blocks take.
 int row_tiles(int m) {
   const int blocks = (m - 1) / kQ8TileM + 1;
   return ((m - 1) / blocks + 64) / 64;
